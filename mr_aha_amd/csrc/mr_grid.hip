@@ -102,11 +102,16 @@ __device__ __forceinline__ int mr_first_point(float x, int nf, int w, double *u_
     return (int)ceil(u - 0.5 * w);
 }
 
+// Element e of the key array is sample r = e mod Nkx of readout s = e div Nkx
+// (trajectory index m = s + Ntrajs r): a stable sort by bin alone then leaves
+// every bin in (readout, position) order. Sorting 32-bit bins takes three
+// digits where (bin, readout, position) keys of 64 bits took eight.
 __global__ void mr_k_grid_keys(const float *traj, long long n, long long Ntrajs, long long Nkx,
-                               mr_grid g, unsigned long long *keys, int *vals)
+                               mr_grid g, unsigned *keys, int *vals)
 {
-    const long long m = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= n) return;
+    const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= n) return;
+    const long long s = e / Nkx, r = e - s * Nkx, m = s + Ntrajs * r;
     long long bin = 0, mul = 1;
     for (int a = 0; a < g.d; ++a) {
         double u;
@@ -116,14 +121,12 @@ __global__ void mr_k_grid_keys(const float *traj, long long n, long long Ntrajs,
         bin += mul * (i0 / g.bs[a]);
         mul *= g.nb[a];
     }
-    const long long s = m % Ntrajs, r = m / Ntrajs;
-    keys[m] = (unsigned long long)bin * (unsigned long long)n + (unsigned long long)(s * Nkx + r);
-    vals[m] = (int)m;
+    keys[e] = (unsigned)bin;
+    vals[e] = (int)m;
 }
 
 __global__ void mr_k_grid_fill(const float *traj, long long n, long long Ntrajs, mr_grid g,
-                               const unsigned long long *keys, const int *perm, int *i0o, int *rd,
-                               double *wt, int *bin_lo, int *bin_hi)
+                               const int *perm, int *i0o, int *rd, double *wt)
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -139,9 +142,89 @@ __global__ void mr_k_grid_fill(const float *traj, long long n, long long Ntrajs,
     }
     for (int a = g.d; a < 3; ++a) i0o[i * 3 + a] = 0;
     rd[i] = (int)(m % Ntrajs);
-    const unsigned long long b = keys[i] / (unsigned long long)n;
-    if (i == 0 || keys[i - 1] / (unsigned long long)n != b) bin_lo[b] = (int)i;
-    if (i == n - 1 || keys[i + 1] / (unsigned long long)n != b) bin_hi[b] = (int)(i + 1);
+}
+
+// start[b] = first sorted sample of bin >= b, b = 0 .. nbins (empty bins
+// included, so the samples of bins b0 .. b1 are start[b0] .. start[b1 + 1]).
+__global__ void mr_k_grid_starts(const unsigned *keys, long long n, long long nbins, int *start)
+{
+    const long long b = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (b > nbins) return;
+    long long lo = 0, hi = n;
+    while (lo < hi) {
+        const long long mid = (lo + hi) >> 1;
+        if ((long long)keys[mid] < b) lo = mid + 1;
+        else hi = mid;
+    }
+    start[b] = (int)lo;
+}
+
+// Candidate samples of a tile (one bin's points): the samples of the bins
+// whose first points reach it, nbr bins back along every axis (each bin
+// once, also where the grid has no more bins than that). Bins that neighbour
+// along x are neighbours in the sorted order, so a row of them is one range,
+// or two where it wraps. Range r of 2 * rows: row r / 2, piece r % 2.
+__device__ __forceinline__ int mr_tile_rows(const mr_grid &g, int *n1, int *n2)
+{
+    const int k1 = (g.d > 1) ? (g.w - 1 + g.bs[1] - 1) / g.bs[1] + 1 : 1;
+    const int k2 = (g.d > 2) ? (g.w - 1 + g.bs[2] - 1) / g.bs[2] + 1 : 1;
+    *n1 = k1 < g.nb[1] ? k1 : g.nb[1];
+    *n2 = k2 < g.nb[2] ? k2 : g.nb[2];
+    return *n1 * *n2;
+}
+
+__device__ __forceinline__ void mr_tile_range(const mr_grid &g, const int *start, const int *t,
+                                              int n1, int r, int *lo, int *hi)
+{
+    const int row = r >> 1;
+    int b1 = t[1] - row % n1, b2 = t[2] - row / n1;
+    if (b1 < 0) b1 += g.nb[1];
+    if (b2 < 0) b2 += g.nb[2];
+    const long long B = (long long)g.nb[0] * (b1 + (long long)g.nb[1] * b2);
+    int k0 = (g.w - 1 + g.bs[0] - 1) / g.bs[0] + 1;
+    if (k0 > g.nb[0]) k0 = g.nb[0];
+    const int x0 = t[0] - k0 + 1;   // first bin of the row, negative when it wraps
+    int f, l;                       // bins f .. l of this piece
+    if ((r & 1) == 0) {
+        f = x0 < 0 ? 0 : x0;
+        l = t[0];
+    } else {
+        f = x0 < 0 ? x0 + g.nb[0] : 0;
+        l = x0 < 0 ? g.nb[0] - 1 : -1;
+    }
+    *lo = (l < f) ? 0 : start[B + f];
+    *hi = (l < f) ? 0 : start[B + l + 1];
+}
+
+__device__ __forceinline__ void mr_tile_of(const mr_grid &g, long long tile, int *t)
+{
+    t[0] = (int)(tile % g.nb[0]);
+    t[1] = (int)((tile / g.nb[0]) % g.nb[1]);
+    t[2] = (int)(tile / ((long long)g.nb[0] * g.nb[1]));
+}
+
+// ext[tile] = segments of MR_GRID_SEG candidates beyond the tile's first
+__global__ void mr_k_grid_segments(mr_grid g, const int *start, int *ext)
+{
+    const long long tile = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (tile >= g.nbins) return;
+    int t[3], n1, n2, cand = 0;
+    mr_tile_of(g, tile, t);
+    const int nr = 2 * mr_tile_rows(g, &n1, &n2);
+    for (int r = 0; r < nr; ++r) {
+        int lo, hi;
+        mr_tile_range(g, start, t, n1, r, &lo, &hi);
+        cand += hi - lo;
+    }
+    ext[tile] = cand > MR_GRID_SEG ? (cand + MR_GRID_SEG - 1) / MR_GRID_SEG - 1 : 0;
+}
+
+// ext_tile / ext_no of every extra segment, from the exclusive sums of ext
+__global__ void mr_k_grid_ext_list(long long nbins, const int *ext, const int *base, int2 *list)
+{
+    const long long tile = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (tile >= nbins) return;
+    for (int k = 0; k < ext[tile]; ++k) list[base[tile] + k] = make_int2((int)tile, k + 1);
 }
 
 void mr_grid_samples_free(mr_grid_samples *s)
@@ -149,76 +232,95 @@ void mr_grid_samples_free(mr_grid_samples *s)
     if (s->i0) (void)hipFree(s->i0);
     if (s->rd) (void)hipFree(s->rd);
     if (s->wt) (void)hipFree(s->wt);
-    if (s->bin_lo) (void)hipFree(s->bin_lo);
-    if (s->bin_hi) (void)hipFree(s->bin_hi);
-    if (s->perm) (void)hipFree(s->perm);
+    if (s->start) (void)hipFree(s->start);
+    if (s->ext) (void)hipFree(s->ext);
     *s = mr_grid_samples();
 }
 
 int mr_grid_samples_build(const mr_grid &g, const float *traj, long long Ntrajs, long long Nkx,
-                          int ndim, hipStream_t stream, mr_grid_samples *out)
+                          hipStream_t stream, mr_grid_samples *out)
 {
-    (void)ndim;
     const long long n = Ntrajs * Nkx;
     MR_REQUIRE(n > 0 && n < 0x7fffffffLL, "gridding: %lld samples outside [1, 2^31)", n);
     MR_REQUIRE(g.nbins < 0x7fffffffLL, "gridding: too many bins (%lld)", g.nbins);
     mr_grid_samples s;
     s.n = n;
-    unsigned long long *keys = nullptr, *keys2 = nullptr;
-    int *vals = nullptr;
+    unsigned *keys = nullptr, *keys2 = nullptr;
+    int *vals = nullptr, *perm = nullptr, *ext = nullptr, *base = nullptr;
     void *tmp = nullptr;
-    size_t tmp_bytes = 0;
+    size_t sort_bytes = 0, scan_bytes = 0;
     hipError_t e = hipSuccess;
+    int end_bit = 1;
+    while (end_bit < 32 && (g.nbins >> end_bit) != 0) ++end_bit;
 #define MR_GA(ptr, bytes) if (e == hipSuccess) e = hipMalloc((void **)&(ptr), (bytes))
-    MR_GA(keys, n * sizeof(unsigned long long));
-    MR_GA(keys2, n * sizeof(unsigned long long));
+    MR_GA(keys, n * sizeof(unsigned));
+    MR_GA(keys2, n * sizeof(unsigned));
     MR_GA(vals, n * sizeof(int));
-    MR_GA(s.perm, n * sizeof(int));
+    MR_GA(perm, n * sizeof(int));
+    MR_GA(ext, (g.nbins + 1) * sizeof(int));
+    MR_GA(base, (g.nbins + 1) * sizeof(int));
     MR_GA(s.i0, n * 3 * sizeof(int));
     MR_GA(s.rd, n * sizeof(int));
     MR_GA(s.wt, (size_t)n * g.d * g.w * sizeof(double));
-    MR_GA(s.bin_lo, g.nbins * sizeof(int));
-    MR_GA(s.bin_hi, g.nbins * sizeof(int));
-#undef MR_GA
+    MR_GA(s.start, (g.nbins + 1) * sizeof(int));
+    if (e == hipSuccess)
+        e = hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, keys, keys2, vals, perm,
+                                              (int)n, 0, end_bit, stream);
+    if (e == hipSuccess)
+        e = hipcub::DeviceScan::ExclusiveSum(nullptr, scan_bytes, ext, base, (int)g.nbins + 1,
+                                             stream);
+    const size_t tmp_bytes = sort_bytes > scan_bytes ? sort_bytes : scan_bytes;
+    MR_GA(tmp, tmp_bytes ? tmp_bytes : 1);
     int rc = MR_SUCCESS;
     if (e != hipSuccess) {
         (void)hipGetLastError();
         mr_set_error("gridding: failed to allocate the sample tables for %lld samples", n);
         rc = MR_ERR_ALLOC;
     }
-    unsigned long long maxkey = (unsigned long long)g.nbins * (unsigned long long)n;
-    int end_bit = 1;
-    while (end_bit < 64 && (maxkey >> end_bit) != 0) ++end_bit;
     if (rc == MR_SUCCESS) {
-        hipLaunchKernelGGL(mr_k_grid_keys, dim3((unsigned)mr_ceil_div(n, 256)), dim3(256), 0,
-                           stream, traj, n, Ntrajs, Nkx, g, keys, vals);
+        const unsigned nblk = (unsigned)mr_ceil_div(n, 256);
+        const unsigned bblk = (unsigned)mr_ceil_div(g.nbins + 1, 256);
+        int total = 0;
+        hipLaunchKernelGGL(mr_k_grid_keys, dim3(nblk), dim3(256), 0, stream, traj, n, Ntrajs, Nkx,
+                           g, keys, vals);
+        size_t bytes = sort_bytes;
         e = hipGetLastError();
         if (e == hipSuccess)
-            e = hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, keys, keys2, vals, s.perm,
-                                                  (int)n, 0, end_bit, stream);
-        if (e == hipSuccess) e = hipMalloc(&tmp, tmp_bytes ? tmp_bytes : 1);
-        if (e == hipSuccess)
-            e = hipcub::DeviceRadixSort::SortPairs(tmp, tmp_bytes, keys, keys2, vals, s.perm,
-                                                  (int)n, 0, end_bit, stream);
-        if (e == hipSuccess) e = hipMemsetAsync(s.bin_lo, 0, g.nbins * sizeof(int), stream);
-        if (e == hipSuccess) e = hipMemsetAsync(s.bin_hi, 0, g.nbins * sizeof(int), stream);
+            e = hipcub::DeviceRadixSort::SortPairs(tmp, bytes, keys, keys2, vals, perm, (int)n, 0,
+                                                  end_bit, stream);
         if (e == hipSuccess) {
-            hipLaunchKernelGGL(mr_k_grid_fill, dim3((unsigned)mr_ceil_div(n, 256)), dim3(256), 0,
-                               stream, traj, n, Ntrajs, g, keys2, s.perm, s.i0, s.rd, s.wt,
-                               s.bin_lo, s.bin_hi);
+            hipLaunchKernelGGL(mr_k_grid_fill, dim3(nblk), dim3(256), 0, stream, traj, n, Ntrajs,
+                               g, perm, s.i0, s.rd, s.wt);
+            hipLaunchKernelGGL(mr_k_grid_starts, dim3(bblk), dim3(256), 0, stream, keys2, n,
+                               g.nbins, s.start);
+            hipLaunchKernelGGL(mr_k_grid_segments, dim3(bblk), dim3(256), 0, stream, g, s.start,
+                               ext);
             e = hipGetLastError();
         }
+        bytes = scan_bytes;   // the sum over all tiles lands in base[nbins]
+        if (e == hipSuccess)
+            e = hipcub::DeviceScan::ExclusiveSum(tmp, bytes, ext, base, (int)g.nbins + 1, stream);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(&total, base + g.nbins, sizeof(int), hipMemcpyDeviceToHost, stream);
         if (e == hipSuccess) e = hipStreamSynchronize(stream);
+        if (e == hipSuccess && total > 0) {
+            s.next = total;
+            e = hipMalloc((void **)&s.ext, (size_t)total * sizeof(int2));
+            if (e == hipSuccess) {
+                hipLaunchKernelGGL(mr_k_grid_ext_list, dim3(bblk), dim3(256), 0, stream, g.nbins,
+                                   ext, base, s.ext);
+                e = hipGetLastError();
+            }
+            if (e == hipSuccess) e = hipStreamSynchronize(stream);
+        }
         if (e != hipSuccess) {
             (void)hipGetLastError();
             mr_set_error("gridding: sample sort failed: %s", hipGetErrorString(e));
             rc = MR_ERR_CUFINUFFT;
         }
     }
-    if (tmp) (void)hipFree(tmp);
-    if (keys) (void)hipFree(keys);
-    if (keys2) (void)hipFree(keys2);
-    if (vals) (void)hipFree(vals);
+    void *scratch[] = {tmp, keys, keys2, vals, perm, ext, base};
+    for (void *p : scratch) if (p) (void)hipFree(p);
     if (rc != MR_SUCCESS) {
         mr_grid_samples_free(&s);
         return rc;
@@ -228,154 +330,261 @@ int mr_grid_samples_build(const mr_grid &g, const float *traj, long long Ntrajs,
 }
 
 // ---------------------------------------------------------------------------
-// Type-1 gather spreading. One 64-lane workgroup per bin-sized tile of the
-// fine grid (8x8 in 2D, 4x4x4 in 3D); lane = fine point. Samples of the
-// candidate bins are staged in LDS 64 at a time and every lane adds its
-// kernel weight. With readout-constant strengths (PER_SAMPLE false) the
-// weights of consecutive samples of one readout are summed first and the
-// CB strengths are applied once per readout run.
+// Type-1 gather spreading. One wavefront per segment of at most MR_GRID_SEG
+// candidate samples of a tile (8x8 points in 2D, 4x4x4 in 3D; lane = fine
+// point). The candidates are taken 64 at a time: lane i tests whether sample i
+// reaches the tile and, if so, stages its kernel values at the tile's points
+// along each axis (zero outside its support), so a lane's weight of a sample
+// is a product of D values read from LDS with no test. With readout-constant
+// strengths (PER_SAMPLE false) the weights of consecutive samples of one
+// readout are summed first and the CB strengths applied once per run; the
+// strengths of a key are contiguous and uniform over the wavefront, so they
+// come through the scalar cache. The first segment of a tile is stored to the
+// fine grid, later ones to `part`, which mr_k_spread_sum adds in order.
+//
+// The bound is the FP64 arithmetic of the weights and strengths once the work
+// is even. A tile at the centre of radial samples has a thousand times the
+// candidates of one at the edge, and with one wavefront per tile the whole
+// pass waited for it. Measured, one wavefront per tile and now: 256x256 L=8
+// (512 x 512 samples, 36 sets) 2.58 -> 0.34 ms, 192x192x32 L=8 (1152 sets)
+// 26.9 -> 3.8 ms, of which the 10.9 GB of output take 2.0, 96^3 L=4 (4000 x
+// 192 samples) 49.7 -> 3.8 ms (9.1 GB, 1.7 ms); per sample, 128 x 384 samples
+// onto 768x768, 4 sets, 1.26 -> 0.09 ms.
 // ---------------------------------------------------------------------------
 
+// LDS of one wavefront: 64 samples' kernel values (the odd stride keeps the
+// staging writes off each other's banks), their keys, and the tile's ranges.
+template <int D> struct mr_spread_lds {
+    static constexpr int BS = (D == 2) ? 8 : 4;
+    static constexpr int STR = D * BS + 1;
+    double w[64 * STR];
+    int key[64];
+    int base[64], end[64];
+};
+
 template <int D, int CB, bool PER_SAMPLE>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(256, 4)
 mr_k_spread(mr_grid g, const int *__restrict__ i0s, const int *__restrict__ rds,
-            const double *__restrict__ wts, const int *__restrict__ perm,
-            const int *__restrict__ bin_lo, const int *__restrict__ bin_hi,
-            const double2 *__restrict__ str, long long sstride, int Q, double2 *__restrict__ fine)
+            const double *__restrict__ wts, const int *__restrict__ start,
+            const int2 *__restrict__ ext, long long next, const double2 *__restrict__ str, int qs,
+            int q0, int Q, double2 *__restrict__ fine, double2 *__restrict__ part)
 {
-    __shared__ int sh_i0[64][3];
-    __shared__ int sh_key[64];
-    __shared__ double sh_w[64][D][MR_GRID_MAXW];
-    const int lane = threadIdx.x;
-    long long tile = blockIdx.x;
-    int t[3], p[3];
-    t[0] = (int)(tile % g.nb[0]);
-    t[1] = (int)((tile / g.nb[0]) % g.nb[1]);
-    t[2] = (int)(tile / ((long long)g.nb[0] * g.nb[1]));
-    if (D == 2) { p[0] = lane & 7; p[1] = lane >> 3; p[2] = 0; }
-    else { p[0] = lane & 3; p[1] = (lane >> 2) & 3; p[2] = lane >> 4; }
-    int gp[3];
-    for (int a = 0; a < 3; ++a) gp[a] = t[a] * g.bs[a] + p[a];
-    const int q0 = blockIdx.y * CB;
-    const int nq = (Q - q0 < CB) ? Q - q0 : CB;
+    using lds_t = mr_spread_lds<D>;
+    constexpr int BS = lds_t::BS, STR = lds_t::STR;
+    __shared__ lds_t sh4[4];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    lds_t &sh = sh4[wave];
+    const long long id = (long long)blockIdx.x * 4 + wave;
+    if (id >= g.nbins + next) return;   // the wavefronts share nothing
+    // extra segments first: they belong to the crowded tiles
+    const int2 es = id < next ? ext[id] : make_int2((int)(id - next), 0);
+    const int seg = __builtin_amdgcn_readfirstlane(es.y);
+    const long long tile = __builtin_amdgcn_readfirstlane(es.x);
+    int t[3], T0[3], p[3], n1, n2;
+    mr_tile_of(g, tile, t);
+    p[0] = lane % BS;
+    p[1] = (lane / BS) % BS;
+    p[2] = (D == 3) ? lane / (BS * BS) : 0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) T0[a] = t[a] * g.bs[a];
     const int w = g.w;
+    const int qb = blockIdx.y * CB;
+
+    // ranges of candidates, inclusive sums of their lengths (2 * rows <= 50)
+    const int nr = 2 * mr_tile_rows(g, &n1, &n2);
+    int lo = 0, hi = 0;
+    if (lane < nr) mr_tile_range(g, start, t, n1, lane, &lo, &hi);
+    int sum = hi - lo;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(sum, o);
+        if (lane >= o) sum += v;
+    }
+    sh.end[lane] = sum;
+    sh.base[lane] = hi - sum;   // candidate k of range r is sample base[r] + k
+    const int total = __builtin_amdgcn_readlane(sum, 63);
+    const int k_end = (seg + 1) * MR_GRID_SEG < total ? (seg + 1) * MR_GRID_SEG : total;
 
     double2 acc[CB];
 #pragma unroll
     for (int q = 0; q < CB; ++q) acc[q] = make_double2(0.0, 0.0);
-    double wsum = 0.0;
-    int cur = -1;
+    const double2 *strq = str + q0 + qb;
 
-    int nbr[3];
-    for (int a = 0; a < 3; ++a) nbr[a] = (a < D) ? (w - 1 + g.bs[a] - 1) / g.bs[a] : 0;
-    for (int k2 = nbr[2]; k2 >= 0; --k2)
-    for (int k1 = nbr[1]; k1 >= 0; --k1)
-    for (int k0 = nbr[0]; k0 >= 0; --k0) {
-        const int b0 = (t[0] - k0 + g.nb[0] * 4) % g.nb[0];
-        const int b1 = (t[1] - k1 + g.nb[1] * 4) % g.nb[1];
-        const int b2 = (t[2] - k2 + g.nb[2] * 4) % g.nb[2];
-        const long long B = b0 + (long long)g.nb[0] * (b1 + (long long)g.nb[1] * b2);
-        const int lo = bin_lo[B], hi = bin_hi[B];
-        for (int base = lo; base < hi; base += 64) {
-            const int cnt = (hi - base < 64) ? hi - base : 64;
-            __syncthreads();
-            if (lane < cnt) {
-                const long long i = base + lane;
-                for (int a = 0; a < 3; ++a) sh_i0[lane][a] = i0s[i * 3 + a];
-                sh_key[lane] = PER_SAMPLE ? perm[i] : rds[i];
-                for (int a = 0; a < D; ++a)
-                    for (int k = 0; k < w; ++k) sh_w[lane][a][k] = wts[(i * D + a) * w + k];
+    for (int k0 = seg * MR_GRID_SEG; k0 < k_end; k0 += 64) {
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const int k = k0 + lane;
+        bool in = k < k_end;
+        int i = 0, o0[D];
+        if (in) {
+            int r = 0;
+#pragma unroll
+            for (int b = 32; b > 0; b >>= 1)
+                if (r + b <= 64 && sh.end[r + b - 1] <= k) r += b;
+            i = sh.base[r] + k;
+#pragma unroll
+            for (int a = 0; a < D; ++a) {
+                int o = T0[a] - i0s[(long long)i * 3 + a];
+                if (o < 0) o += g.nf[a];
+                o0[a] = o;
+                in = in && (o < w || o + BS > g.nf[a]);
             }
-            __syncthreads();
-            for (int j = 0; j < cnt; ++j) {
-                double wv = 1.0;
-                bool in = true;
+        }
+        const unsigned long long m = __ballot(in);
+        const int cnt = __popcll(m);
+        if (in) {
+            const int slot = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                                       __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+            double *ws = sh.w + slot * STR;
+            sh.key[slot] = PER_SAMPLE ? i : rds[i];
 #pragma unroll
-                for (int a = 0; a < D; ++a) {
-                    int o = gp[a] - sh_i0[j][a];
-                    if (o < 0) o += g.nf[a];
-                    in = in && (o < w);
-                    wv *= in ? sh_w[j][a][in ? o : 0] : 0.0;
+            for (int a = 0; a < D; ++a) {
+                const double *wt = wts + ((long long)i * D + a) * w;
+#pragma unroll
+                for (int b = 0; b < BS; ++b) {
+                    int o = o0[a] + b;
+                    if (o >= g.nf[a]) o -= g.nf[a];
+                    ws[a * BS + b] = (o < w) ? wt[o] : 0.0;
                 }
-                if (!in) wv = 0.0;
-                const int key = sh_key[j];
-                if (PER_SAMPLE) {
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const int key = sh.key[lane];
+        auto weight = [&](int j) {
+            const double *ws = sh.w + j * STR;
+            double v = ws[p[0]] * ws[BS + p[1]];
+            if (D == 3) v *= ws[2 * BS + p[2]];
+            return v;
+        };
+        auto apply = [&](double wv, int ky) {
+            const double2 *c = strq + (long long)ky * qs;
 #pragma unroll
-                    for (int q = 0; q < CB; ++q)
-                        if (q < nq) {
-                            const double2 c = str[(long long)(q0 + q) * sstride + key];
-                            acc[q].x += wv * c.x;
-                            acc[q].y += wv * c.y;
-                        }
-                } else {
-                    if (key != cur) {
-                        if (cur >= 0) {
+            for (int q = 0; q < CB; ++q) {
+                const double2 v = c[q];
+                acc[q].x += wv * v.x;
+                acc[q].y += wv * v.y;
+            }
+        };
+        // last sample of every run of one readout
+        unsigned long long ends = ~0ULL;
+        if (!PER_SAMPLE) {
+            const int nxt = __shfl_down(key, 1);
+            ends = __ballot(lane == cnt - 1 || nxt != key);
+        }
+        // eight weights at a time, so that their LDS reads overlap
+        double wsum = 0.0;
+        for (int j0 = 0; j0 < cnt; j0 += 8) {
+            double wv[8];
 #pragma unroll
-                            for (int q = 0; q < CB; ++q)
-                                if (q < nq) {
-                                    const double2 c = str[(long long)(q0 + q) * sstride + cur];
-                                    acc[q].x += wsum * c.x;
-                                    acc[q].y += wsum * c.y;
-                                }
-                        }
-                        cur = key;
-                        wsum = 0.0;
-                    }
-                    wsum += wv;
+            for (int j = 0; j < 8; ++j) wv[j] = weight((j0 + j) & 63);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                if (j0 + j >= cnt) break;
+                wsum += wv[j];
+                if ((ends >> (j0 + j)) & 1) {
+                    apply(wsum, __builtin_amdgcn_readlane(key, j0 + j));
+                    wsum = 0.0;
                 }
             }
         }
     }
-    if (!PER_SAMPLE && cur >= 0) {
-#pragma unroll
-        for (int q = 0; q < CB; ++q)
-            if (q < nq) {
-                const double2 c = str[(long long)(q0 + q) * sstride + cur];
-                acc[q].x += wsum * c.x;
-                acc[q].y += wsum * c.y;
-            }
+    double2 *dst;
+    long long qstride;
+    if (id < next) {
+        dst = part + id * 64 + lane;
+        qstride = next * 64;
+    } else {
+        dst = fine + (T0[0] + p[0]) +
+              (long long)g.nf[0] * ((T0[1] + p[1]) + (long long)g.nf[1] * (T0[2] + p[2]));
+        qstride = g.nfine;
     }
-    if (gp[0] < g.nf[0] && gp[1] < g.nf[1] && gp[2] < g.nf[2]) {
-        const long long gl = gp[0] + (long long)g.nf[0] * (gp[1] + (long long)g.nf[1] * gp[2]);
 #pragma unroll
-        for (int q = 0; q < CB; ++q)
-            if (q < nq) fine[(long long)(q0 + q) * g.nfine + gl] = acc[q];
-    }
+    for (int q = 0; q < CB; ++q)
+        if (qb + q < Q) dst[(long long)(qb + q) * qstride] = acc[q];
 }
 
-template <bool PER_SAMPLE>
-static int mr_spread_launch(const mr_grid &g, const mr_grid_samples &s, const double2 *str,
-                            long long sstride, int Q, double2 *fine, hipStream_t stream)
+// Add the extra segments of every crowded tile to its first: the workgroup
+// of a tile's first extra segment (number 1) takes them all, in order.
+template <int D>
+__global__ void __launch_bounds__(64)
+mr_k_spread_sum(mr_grid g, const int2 *__restrict__ ext, long long next,
+                const double2 *__restrict__ part, double2 *__restrict__ fine)
 {
-    constexpr int CB = 16;
-    const dim3 grid((unsigned)g.nbins, (unsigned)((Q + CB - 1) / CB));
-    if (g.d == 2)
-        hipLaunchKernelGGL((mr_k_spread<2, CB, PER_SAMPLE>), grid, dim3(64), 0, stream, g, s.i0,
-                           s.rd, s.wt, s.perm, s.bin_lo, s.bin_hi, str, sstride, Q, fine);
-    else
-        hipLaunchKernelGGL((mr_k_spread<3, CB, PER_SAMPLE>), grid, dim3(64), 0, stream, g, s.i0,
-                           s.rd, s.wt, s.perm, s.bin_lo, s.bin_hi, str, sstride, Q, fine);
+    constexpr int BS = mr_spread_lds<D>::BS;
+    const long long e0 = blockIdx.x;
+    const int2 es = ext[e0];
+    if (es.y != 1) return;
+    long long e1 = e0 + 1;
+    while (e1 < next && ext[e1].x == es.x) ++e1;
+    const int lane = threadIdx.x;
+    int t[3];
+    mr_tile_of(g, es.x, t);
+    const long long gl = (t[0] * BS + lane % BS) +
+                         (long long)g.nf[0] * ((t[1] * BS + (lane / BS) % BS) +
+                                               (long long)g.nf[1] *
+                                                   (D == 3 ? t[2] * BS + lane / (BS * BS) : 0));
+    double2 *f = fine + (long long)blockIdx.y * g.nfine + gl;
+    const double2 *s = part + (long long)blockIdx.y * next * 64 + lane;
+    double2 a = *f;
+#pragma unroll 8
+    for (long long e = e0; e < e1; ++e) {
+        const double2 v = s[e * 64];
+        a.x += v.x;
+        a.y += v.y;
+    }
+    *f = a;
+}
+
+template <int D, bool PER_SAMPLE>
+static int mr_spread_launch(const mr_grid &g, const mr_grid_samples &s, const double2 *str, int qs,
+                            int q0, int Q, double2 *fine, double2 *part, hipStream_t stream)
+{
+    // strengths per wavefront: the fewest that keep the number of chunks of 16
+    const int chunks = (Q + 15) / 16, per = (Q + chunks - 1) / chunks;
+    const long long blocks = mr_ceil_div(g.nbins + s.next, 4);
+#define MR_SPREAD(CB)                                                                             \
+    do {                                                                                          \
+        MR_GRID_CHECK(blocks, 256, "mr_k_spread");                                                \
+        hipLaunchKernelGGL((mr_k_spread<D, CB, PER_SAMPLE>),                                      \
+                           dim3((unsigned)blocks, (unsigned)((Q + CB - 1) / CB)), dim3(256), 0,   \
+                           stream, g, s.i0, s.rd, s.wt, s.start, s.ext, s.next, str, qs, q0, Q,   \
+                           fine, part);                                                           \
+    } while (0)
+    if (per <= 4) MR_SPREAD(4);
+    else if (per <= 8) MR_SPREAD(8);
+    else if (per <= 12) MR_SPREAD(12);
+    else MR_SPREAD(16);
+#undef MR_SPREAD
     MR_LAUNCH_CHECK("mr_k_spread");
+    if (s.next > 0) {
+        hipLaunchKernelGGL(mr_k_spread_sum<D>, dim3((unsigned)s.next, (unsigned)Q), dim3(64), 0,
+                           stream, g, s.ext, s.next, part, fine);
+        MR_LAUNCH_CHECK("mr_k_spread_sum");
+    }
     return MR_SUCCESS;
 }
 
-int mr_grid_spread(const mr_grid &g, const mr_grid_samples &s, const double2 *str,
-                   long long Ntrajs, int Q, double2 *fine, hipStream_t stream)
+int mr_grid_spread(const mr_grid &g, const mr_grid_samples &s, const double2 *str, int qs, int q0,
+                   int Q, double2 *fine, double2 *part, hipStream_t stream)
 {
-    return mr_spread_launch<false>(g, s, str, Ntrajs, Q, fine, stream);
+    return g.d == 2 ? mr_spread_launch<2, false>(g, s, str, qs, q0, Q, fine, part, stream)
+                    : mr_spread_launch<3, false>(g, s, str, qs, q0, Q, fine, part, stream);
 }
 
 int mr_grid_spread_samples(const mr_grid &g, const mr_grid_samples &s, const double2 *str, int Q,
-                           double2 *fine, hipStream_t stream)
+                           double2 *fine, double2 *part, hipStream_t stream)
 {
-    return mr_spread_launch<true>(g, s, str, s.n, Q, fine, stream);
+    return g.d == 2 ? mr_spread_launch<2, true>(g, s, str, Q, 0, Q, fine, part, stream)
+                    : mr_spread_launch<3, true>(g, s, str, Q, 0, Q, fine, part, stream);
 }
 
 // Type-2 interpolation, one thread per (sorted sample, set q).
 template <int D>
 __global__ void mr_k_interp(mr_grid g, const int *__restrict__ i0s, const double *__restrict__ wts,
-                            const int *__restrict__ perm, long long n, const double2 *__restrict__ fine,
-                            int Q, double2 *__restrict__ out)
+                            long long n, const double2 *__restrict__ fine, int Q,
+                            double2 *__restrict__ out)
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const int q = blockIdx.y;
@@ -411,7 +620,7 @@ __global__ void mr_k_interp(mr_grid g, const int *__restrict__ i0s, const double
             }
         }
     }
-    out[(long long)q * n + perm[i]] = make_double2(ar, ai);
+    out[i * Q + q] = make_double2(ar, ai);
 }
 
 int mr_grid_interp(const mr_grid &g, const mr_grid_samples &s, const double2 *fine, int Q,
@@ -419,11 +628,9 @@ int mr_grid_interp(const mr_grid &g, const mr_grid_samples &s, const double2 *fi
 {
     const dim3 grid((unsigned)mr_ceil_div(s.n, 256), (unsigned)Q);
     if (g.d == 2)
-        hipLaunchKernelGGL(mr_k_interp<2>, grid, dim3(256), 0, stream, g, s.i0, s.wt, s.perm, s.n,
-                           fine, Q, out);
+        hipLaunchKernelGGL(mr_k_interp<2>, grid, dim3(256), 0, stream, g, s.i0, s.wt, s.n, fine, Q, out);
     else
-        hipLaunchKernelGGL(mr_k_interp<3>, grid, dim3(256), 0, stream, g, s.i0, s.wt, s.perm, s.n,
-                           fine, Q, out);
+        hipLaunchKernelGGL(mr_k_interp<3>, grid, dim3(256), 0, stream, g, s.i0, s.wt, s.n, fine, Q, out);
     MR_LAUNCH_CHECK("mr_k_interp");
     return MR_SUCCESS;
 }

@@ -36,35 +36,50 @@ void mr_grid_setup(mr_grid *g, int d, const int *M, double eps);
 // natural order (index j <-> delta = j or j - M). Host vector.
 std::vector<double> mr_grid_deconv(const mr_grid &g, int a);
 
+// Candidate samples per segment of mr_k_spread: a wavefront's share of a tile.
+// Large enough that few tiles are split (each extra segment costs a partial
+// tile per strength set in memory), small enough that the last wavefront ends
+// with the others (1024: the per-sample launch of a 192x192 comparator takes
+// 0.31 ms instead of 0.09, a 256x256 L=8 build's 0.53 instead of 0.34).
+#define MR_GRID_SEG 256
+
+// Strength rows are read in chunks of up to this many sets, also past the
+// last set of a row: the strength array ends with as many spare entries.
+#define MR_GRID_STR_PAD 16
+
 // Per-sample geometry, sorted by (bin, readout, readout position).
 struct mr_grid_samples {
     long long n = 0;        // samples
     int *i0 = nullptr;      // [n * 3] first fine point per axis (mod nf), sorted order
     int *rd = nullptr;      // [n] readout of each sorted sample
     double *wt = nullptr;   // [n * d * w] weights per axis, sorted order
-    int *bin_lo = nullptr;  // [nbins] first sorted sample of each bin
-    int *bin_hi = nullptr;  // [nbins] one past the last
-    int *perm = nullptr;    // [n] original sample index of each sorted sample
+    int *start = nullptr;   // [nbins + 1] first sorted sample of bin >= b
+    long long next = 0;     // segments beyond the first of their tile
+    int2 *ext = nullptr;    // [next] (tile, segment number >= 1), ascending
+    // scratch values (double2) that spreading Q sets needs for them
+    long long part_elems(long long Q) const { return next * 64 * Q; }
 };
 
 // Build the sorted sample table from a [Ntrajs, Nkx, ndim] trajectory
 // (first `g.d` coordinates used) on `stream`. Synchronous.
 int mr_grid_samples_build(const mr_grid &g, const float *traj, long long Ntrajs, long long Nkx,
-                          int ndim, hipStream_t stream, mr_grid_samples *out);
+                          hipStream_t stream, mr_grid_samples *out);
 void mr_grid_samples_free(mr_grid_samples *s);
 
-// Type-1 spreading of Q strength sets (strength of sample m, set q:
-// str[q * Ntrajs + readout(m)], i.e. constant along a readout) onto Q fine
+// Type-1 spreading of Q strength sets (strength of a sample of readout s, set
+// q: str[s * qs + q0 + q], i.e. constant along a readout) onto Q fine
 // grids fine[q * nfine + g], complex double. Gather formulation: every fine
-// point sums the samples of the bins that can reach it; no atomics.
-int mr_grid_spread(const mr_grid &g, const mr_grid_samples &s, const double2 *str,
-                   long long Ntrajs, int Q, double2 *fine, hipStream_t stream);
+// point sums the samples of the bins that can reach it; no atomics. `part`
+// holds part_elems(Q) values.
+int mr_grid_spread(const mr_grid &g, const mr_grid_samples &s, const double2 *str, int qs, int q0,
+                   int Q, double2 *fine, double2 *part, hipStream_t stream);
 
-// Same with per-sample strengths str[q * nsamp + m] (m = original index).
+// Same with per-sample strengths str[i * Q + q] of sorted sample i.
 int mr_grid_spread_samples(const mr_grid &g, const mr_grid_samples &s, const double2 *str,
-                           int Q, double2 *fine, hipStream_t stream);
+                           int Q, double2 *fine, double2 *part, hipStream_t stream);
 
-// Type-2 interpolation: out[q * nsamp + m] = sum_points fine[q][p] weight.
+// Type-2 interpolation: out[i * Q + q] = sum_points fine[q][p] weight of
+// sorted sample i.
 int mr_grid_interp(const mr_grid &g, const mr_grid_samples &s, const double2 *fine, int Q,
                    double2 *out, hipStream_t stream);
 

@@ -30,8 +30,9 @@ struct mr_nufft_eng {
     double2 *img;   // [Nimg, L] (z fastest after x, y): image-side work
     double2 *acc;   // [Nimg, L] coil sum
     double2 *fine;  // [Q, nfine]
-    double2 *k1;    // [Q, Mnu]
-    double2 *k2;    // [Q, Mnu]
+    double2 *k1;    // [Mnu (sorted samples)][Q]
+    double2 *k2;    // [Mnu][Q], plus the spare entries of a strength array
+    double2 *part;  // scratch of the spreading
     mr_fft_len<double> fz;
 };
 
@@ -39,7 +40,7 @@ static void mr_nufft_free(mr_nufft_eng *e)
 {
     mr_grid_samples_free(&e->smp);
     for (double *p : e->dc) if (p) (void)hipFree(p);
-    void *bufs[] = {e->phi2, e->img, e->acc, e->fine, e->k1, e->k2};
+    void *bufs[] = {e->phi2, e->img, e->acc, e->fine, e->k1, e->k2, e->part};
     for (void *p : bufs) if (p) (void)hipFree(p);
     delete e;
 }
@@ -70,7 +71,7 @@ int mr_nufft_eng_create(const mr_config *cfg, const mr_complex *d_phi2, const fl
     e->Mnu = Ntrajs * Nkx;
     int modes[3] = {cfg->n_dim[0], cfg->n_dim[1], three ? cfg->n_dim[2] : 1};
     mr_grid_setup(&e->g, e->d, modes, cfg->eps);
-    int rc = mr_grid_samples_build(e->g, d_traj, Ntrajs, Nkx, e->d, e->s, &e->smp);
+    int rc = mr_grid_samples_build(e->g, d_traj, Ntrajs, Nkx, e->s, &e->smp);
     if (rc != MR_SUCCESS) { mr_nufft_free(e); return rc; }
     const size_t phi2_bytes = (size_t)Ntrajs * e->Nkz * cfg->L * cfg->L * sizeof(float2);
     const size_t img_bytes = (size_t)e->Nimg * cfg->L * sizeof(double2);
@@ -79,7 +80,11 @@ int mr_nufft_eng_create(const mr_config *cfg, const mr_complex *d_phi2, const fl
     if (he == hipSuccess) he = hipMalloc((void **)&e->acc, img_bytes);
     if (he == hipSuccess) he = hipMalloc((void **)&e->fine, (size_t)e->Q * e->g.nfine * sizeof(double2));
     if (he == hipSuccess) he = hipMalloc((void **)&e->k1, (size_t)e->Q * e->Mnu * sizeof(double2));
-    if (he == hipSuccess) he = hipMalloc((void **)&e->k2, (size_t)e->Q * e->Mnu * sizeof(double2));
+    if (he == hipSuccess)
+        he = hipMalloc((void **)&e->k2,
+                       ((size_t)e->Q * e->Mnu + MR_GRID_STR_PAD) * sizeof(double2));
+    if (he == hipSuccess && e->smp.next > 0)
+        he = hipMalloc((void **)&e->part, (size_t)e->smp.part_elems(e->Q) * sizeof(double2));
     for (int a = 0; a < 3 && he == hipSuccess; ++a) {
         std::vector<double> dc = mr_grid_deconv(e->g, a);
         he = hipMalloc((void **)&e->dc[a], dc.size() * sizeof(double));
@@ -189,26 +194,25 @@ __global__ void mr_k_nu_crop(const double2 *fine, mr_grid g, long long Nplane, i
     img[id] = make_double2(v.x * w, v.y * w);
 }
 
-// k2[(K + Nkz l), m] = sum_j k1[(K + Nkz j), m] B_{s(m),K}(j, l)
-__global__ void mr_k_nu_gram(const double2 *k1, const float2 *phi2, long long Mnu, long long Ntrajs,
-                             int Nkz, int L, double2 *k2)
+// k2[i, K + Nkz l] = sum_j k1[i, K + Nkz j] B_{rd(i),K}(j, l)
+__global__ void mr_k_nu_gram(const double2 *k1, const float2 *phi2, const int *rd, long long Mnu,
+                             long long Ntrajs, int Nkz, int L, double2 *k2)
 {
     const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (id >= Mnu * Nkz) return;
-    const long long m = id % Mnu;
-    const int K = (int)(id / Mnu);
-    const long long s = m % Ntrajs;
-    const float2 *B = phi2 + s + Ntrajs * (long long)K;  // entry (j,l) at + Ntrajs*Nkz*(j + L*l)
-    const long long bs = Ntrajs * Nkz;
+    const long long i = id / Nkz;
+    const int K = (int)(id - i * Nkz);
+    const float2 *B = phi2 + rd[i] + Ntrajs * (long long)K;  // entry (j,l) at + Ntrajs*Nkz*(j + L*l)
+    const long long bs = Ntrajs * Nkz, row = i * Nkz * L + K;
     for (int l = 0; l < L; ++l) {
         double re = 0.0, im = 0.0;
         for (int j = 0; j < L; ++j) {
-            const double2 v = k1[m + Mnu * (K + (long long)Nkz * j)];
+            const double2 v = k1[row + (long long)Nkz * j];
             const float2 b = B[bs * (j + (long long)L * l)];
             re += v.x * b.x - v.y * b.y;
             im += v.x * b.y + v.y * b.x;
         }
-        k2[m + Mnu * (K + (long long)Nkz * l)] = make_double2(re, im);
+        k2[row + (long long)Nkz * l] = make_double2(re, im);
     }
 }
 
@@ -275,9 +279,9 @@ int mr_nufft_eng_execute(mr_nufft_eng *e, const mr_complex *d_x, const mr_comple
         MR_TRY(mr_grid_fft(e->g, e->fine, nullptr, e->Q, false, e->s));
         MR_TRY(mr_grid_interp(e->g, e->smp, e->fine, e->Q, e->k1, e->s));
         hipLaunchKernelGGL(mr_k_nu_gram, dim3((unsigned)mr_ceil_div(e->Mnu * e->Nkz, 256)), dim3(256),
-                           0, e->s, e->k1, e->phi2, e->Mnu, e->Ntrajs, e->Nkz, L, e->k2);
+                           0, e->s, e->k1, e->phi2, e->smp.rd, e->Mnu, e->Ntrajs, e->Nkz, L, e->k2);
         MR_LAUNCH_CHECK("mr_k_nu_gram");
-        MR_TRY(mr_grid_spread_samples(e->g, e->smp, e->k2, e->Q, e->fine, e->s));
+        MR_TRY(mr_grid_spread_samples(e->g, e->smp, e->k2, e->Q, e->fine, e->part, e->s));
         MR_TRY(mr_grid_fft(e->g, e->fine, nullptr, e->Q, true, e->s));
         hipLaunchKernelGGL(mr_k_nu_crop, dim3((unsigned)mr_ceil_div(Nplane * e->Q, 256)), dim3(256), 0,
                            e->s, e->fine, e->g, Nplane, e->Q, e->dc[0], e->dc[1], e->dc[2], e->img);

@@ -21,8 +21,9 @@
 #include <chrono>
 #include <cstring>
 
-// c[q * Ntrajs + s] = packed element t of the Gram block of readout s and kz
-// plane z (q = z + Nkz t); phi2 is [Ntrajs, Nkz, L, L] column-major
+// c[s * Q + q] = packed element t of the Gram block of readout s and kz
+// plane z (q = z + Nkz t, Q of them: a readout's strengths are contiguous, as
+// the spreading reads them); phi2 is [Ntrajs, Nkz, L, L] column-major
 // (src/cuda/mr_kernels.cu:307-333 packing).
 __global__ void mr_k_pack_strengths(const float2 *phi2, long long Ntrajs, int Nkz, int L,
                                     int upper, int T, double2 *c)
@@ -45,7 +46,7 @@ __global__ void mr_k_pack_strengths(const float2 *phi2, long long Ntrajs, int Nk
         acc += len;
     }
     const float2 v = phi2[s + Ntrajs * (z + (long long)Nkz * (i + (long long)L * j))];
-    c[id] = make_double2((double)v.x, (double)v.y);
+    c[s * T * Nkz + q] = make_double2((double)v.x, (double)v.y);
 }
 
 // nat[j + Ptr*q] = fine[(delta mod nf) + nfine*q] * dc0[jx] dc1[jy] dc2[jz]
@@ -173,7 +174,7 @@ int mr_toep_ifft(const toep_geom &tg, double2 *nat, int Qc, hipStream_t s)
 }
 
 struct toep_bufs {
-    double2 *c = nullptr, *fine = nullptr, *nat = nullptr;
+    double2 *c = nullptr, *fine = nullptr, *nat = nullptr, *part = nullptr;
     double *dc[3] = {nullptr, nullptr, nullptr};
     int *inv = nullptr;
     ~toep_bufs()
@@ -181,6 +182,7 @@ struct toep_bufs {
         if (c) (void)hipFree(c);
         if (fine) (void)hipFree(fine);
         if (nat) (void)hipFree(nat);
+        if (part) (void)hipFree(part);
         for (double *p : dc) if (p) (void)hipFree(p);
         if (inv) (void)hipFree(inv);
     }
@@ -208,19 +210,18 @@ int mr_calc_toep_impl(const mr_config *cfg, const mr_complex *d_phi2, const floa
     const toep_geom tg = mr_toep_geom(cfg);
     const int T = (int)mr_num_tri(cfg->L);
     const long long Q = (long long)T * tg.Nkz;
-    const int ndim = (cfg->traj_type == MR_TRAJ_3D) ? 3 : 2;
 
     mr_grid g;
     mr_grid_setup(&g, tg.d, tg.M, cfg->eps);
     toep_bufs b;
     mr_grid_samples smp;
-    MR_TRY(mr_grid_samples_build(g, d_traj, Ntrajs, Nkx, ndim, s, &smp));
+    MR_TRY(mr_grid_samples_build(g, d_traj, Ntrajs, Nkx, s, &smp));
     struct samples_guard {
         mr_grid_samples *p;
         ~samples_guard() { mr_grid_samples_free(p); }
     } guard{&smp};
 
-    MR_HIP_CHECK(hipMalloc((void **)&b.c, Q * Ntrajs * sizeof(double2)));
+    MR_HIP_CHECK(hipMalloc((void **)&b.c, (Q * Ntrajs + MR_GRID_STR_PAD) * sizeof(double2)));
     hipLaunchKernelGGL(mr_k_pack_strengths, dim3((unsigned)mr_ceil_div(Q * Ntrajs, 256)),
                        dim3(256), 0, s, reinterpret_cast<const float2 *>(d_phi2), (long long)Ntrajs,
                        tg.Nkz, cfg->L, cfg->triangulation == MR_TRI_UPPER ? 1 : 0, T, b.c);
@@ -238,7 +239,7 @@ int mr_calc_toep_impl(const mr_config *cfg, const mr_complex *d_phi2, const floa
     // Chunk of components: fine grids + natural-order grids within budget.
     size_t budget = 0;
     MR_TRY(mr_mem_budget(cfg, &budget));
-    const size_t per_q = ((size_t)g.nfine + (size_t)tg.Ptr) * sizeof(double2);
+    const size_t per_q = ((size_t)g.nfine + (size_t)tg.Ptr + (size_t)smp.part_elems(1)) * sizeof(double2);
     long long Qc = (long long)(budget / 2 / per_q);
     const long long cap = mr_env_ll("MR_AHA_TOEP_MAX_CHUNK", 0);
     if (cap > 0 && Qc > cap) Qc = cap;
@@ -247,6 +248,8 @@ int mr_calc_toep_impl(const mr_config *cfg, const mr_complex *d_phi2, const floa
     if (Qc < 1) Qc = 1;
     hipError_t e = hipMalloc((void **)&b.fine, (size_t)g.nfine * Qc * sizeof(double2));
     if (e == hipSuccess) e = hipMalloc((void **)&b.nat, (size_t)tg.Ptr * Qc * sizeof(double2));
+    if (e == hipSuccess && smp.next > 0)
+        e = hipMalloc((void **)&b.part, (size_t)smp.part_elems(Qc) * sizeof(double2));
     if (e != hipSuccess) {
         (void)hipGetLastError();
         MR_FAIL(MR_ERR_ALLOC,
@@ -256,7 +259,7 @@ int mr_calc_toep_impl(const mr_config *cfg, const mr_complex *d_phi2, const floa
     }
     for (long long q0 = 0; q0 < Q; q0 += Qc) {
         const int qn = (int)((Q - q0 < Qc) ? Q - q0 : Qc);
-        MR_TRY(mr_grid_spread(g, smp, b.c + q0 * Ntrajs, Ntrajs, qn, b.fine, s));
+        MR_TRY(mr_grid_spread(g, smp, b.c, (int)Q, (int)q0, qn, b.fine, b.part, s));
         MR_TRY(mr_grid_fft(g, b.fine, nullptr, qn, false, s));
         MR_GRID_CHECK(mr_ceil_div(tg.Ptr * qn, 256), 256, "mr_k_deconv");
         hipLaunchKernelGGL(mr_k_deconv, dim3((unsigned)mr_ceil_div(tg.Ptr * qn, 256)), dim3(256),
