@@ -10,11 +10,14 @@
 //   1. gather-spread (FP64) of the readout-constant strengths onto the
 //      2x fine grid (mr_grid_spread: no atomics, one strength multiply per
 //      readout run of each bin),
-//   2. forward FFT of the fine grids (FP64, sign -1),
-//   3. deconvolution by the ES kernel's transform and crop to the M modes,
-//      written in natural order,
-//   4. inverse FFT over the M grid (FP64, sign +1),
-//   5. natural -> centered shift, 1/prod M, FP32 store (or mask gather).
+//   2. per axis, in one pass over the pencils (mr_k_toep_axis): forward FFT of
+//      the fine pencil (FP64, sign -1), crop to the M modes and deconvolution
+//      by the ES kernel's transform, inverse FFT over the M modes (sign +1),
+//      centered store; the last axis scales by 1/prod M and stores FP32 (or
+//      gathers the mask).
+// A mode count with a prime factor that has no unrolled butterfly takes step 2
+// as separate passes: FFTs of the fine axes, deconvolution, inverse FFTs of
+// the mode axes, shifted store.
 
 #include "mr_grid.hpp"
 
@@ -114,6 +117,211 @@ __global__ void mr_k_toep_store(const double2 *nat, int m0, int m1, int m2, int 
     if (row >= 0) out[row + nm * t] = o;
 }
 
+// ---------------------------------------------------------------------------
+// One axis of the build in one pass. The forward transform of the fine axis,
+// the crop with its deconvolution weights and the inverse transform of the
+// mode axis act on one axis each, so they commute with those of the other
+// axes and an axis can be finished before the next: a pencil of nf values is
+// read, becomes M centered values in LDS and is written back over its own
+// first M places (the pitch stays that of the fine grid, no second buffer).
+// Later axes then run over M instead of nf values of the finished ones.
+//
+// The bound is memory: 2D moves 16 nf^2 read, 8 nf^2 written and read, 2 nf^2
+// written bytes (and the spread's 16 nf^2) where the separate passes moved
+// three times that. Measured, all separate passes and these: 256x256 L=8 (36
+// components, nf 1024) 1.42 -> 0.55 ms, 192x192x32 L=8 (1152, nf 768) 27.3 ->
+// 9.8 ms, 96^3 L=4 (10, nf 384) 27.1 -> 8.3 ms; 2.7 to 3.3 TB/s along x. The pencils of a workgroup share 8 NT values of LDS
+// (72 KB at 512 work-items: two workgroups per CU); along y and z they are neighbours in
+// x, 64 bytes at nf = 1024, and the tiles that share a line are neighbours on
+// one XCD.
+// ---------------------------------------------------------------------------
+
+#define MR_TA_MAXTX 32
+
+// LDS place of element e: one spare value per 8, so that the radix-8 writes
+// (8 values apart) of neighbouring lanes fall in different banks.
+__host__ __device__ inline int mr_ta_at(int e) { return e + (e >> 3); }
+
+// Pencil p = i + n0 (j + n1 o) starts at s0 i + s1 j + s2 o, elements `es`
+// apart; M of them replace the nf read.
+struct mr_ta_axis {
+    double2 *data;
+    long long n0, n1, s0, s1, s2, es;
+    int shift;   // centering: mode j is stored at (j + shift) mod M
+};
+// Where the last axis stores: value k along it of pencil (i, j, o = q) is
+// centered element i + c1 j + cs k of component q0 + o.
+struct mr_ta_out {
+    float2 *out;
+    const int *inv;   // mask rows, or null
+    long long c1, cs, Ptr, q0, nm;
+    int Nkz;
+    double scale;
+};
+
+// One in-place stage over tp pencils of length n (mr_stage_reg with the padded
+// places). CROP: the first inverse stage, whose inputs are the cropped modes of
+// the fine pencil (length nf) times their deconvolution weights. A butterfly
+// loads its first twiddle and forms the others as products of two lower ones
+// (three roundings deep at most): the texture unit would bind the stage with
+// seven 16-byte twiddle loads beside eight LDS reads.
+template <int RR, bool INV, bool CROP, int NT>
+__device__ __forceinline__ void mr_ta_stage(double2 *A, const double2 *tws, const double *dc,
+                                            int nf, int n, int ns, int tp, int Ns,
+                                            const mr_fdiv &mdv, const mr_fdiv &nsdv)
+{
+    constexpr int EMAX = CROP ? 4 * NT : 8 * NT;   // a crop keeps at most half the pencil
+    constexpr int KMAX = (EMAX / RR + NT - 1) / NT;
+    const int m = n / RR, nb = tp * m, pos = n - n / 2;
+    double2 v[KMAX][RR];
+#pragma unroll
+    for (int k = 0; k < KMAX; ++k) {
+        const int f = threadIdx.x + k * NT;
+        if (f < nb) {
+            const int p = (int)mr_fdiv_q(mdv, (unsigned)f), j = f - p * m;
+            const double2 *a = A + p * ns;
+#pragma unroll
+            for (int r = 0; r < RR; ++r) {
+                const int e = j + r * m;
+                if (CROP) {
+                    const double w = dc[e];
+                    const double2 x = a[mr_ta_at(e < pos ? e : e + nf - n)];
+                    v[k][r] = make_double2(x.x * w, x.y * w);
+                } else {
+                    v[k][r] = a[mr_ta_at(e)];
+                }
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < KMAX; ++k) {
+        const int f = threadIdx.x + k * NT;
+        if (f < nb) {
+            const int p = (int)mr_fdiv_q(mdv, (unsigned)f), j = f - p * m;
+            const int jn = (int)mr_fdiv_q(nsdv, (unsigned)j), kk = j - jn * Ns;
+            if constexpr (RR > 1) {
+                if (Ns > 1) {
+                    double2 w[RR];
+                    w[1] = tws[Ns + kk - 1];
+#pragma unroll
+                    for (int r = 2; r < RR; ++r) w[r] = cmul(w[r / 2], w[r - r / 2]);
+#pragma unroll
+                    for (int r = 1; r < RR; ++r) v[k][r] = INV ? cmulc(w[r], v[k][r]) : cmul(w[r], v[k][r]);
+                }
+                bfly<RR, INV>(v[k]);
+            }
+            double2 *b = A + p * ns;
+            const int o = jn * Ns * RR + kk;
+#pragma unroll
+            for (int q = 0; q < RR; ++q) b[mr_ta_at(o + q * Ns)] = v[k][q];
+        }
+    }
+    __syncthreads();
+}
+
+template <bool INV, bool CROP, int NT>
+__device__ __forceinline__ void mr_ta_stages(double2 *A, const mr_fft_len<double> &f,
+                                             const double *dc, int nf, int s0, int s1, int ns,
+                                             int tp)
+{
+    int Ns = 1;
+    for (int s = 0; s < s1; ++s) {
+        const int RR = f.radix[s];
+        const mr_fdiv &md = f.mdiv[s], &nd = f.nsdiv[s];
+#define MR_TA_ST(R)                                                                               \
+    case R: mr_ta_stage<R, INV, CROP, NT>(A, f.tws, dc, nf, f.n, ns, tp, Ns, md, nd); break;
+        if (s >= s0) {
+            switch (RR) {
+                MR_TA_ST(2) MR_TA_ST(3) MR_TA_ST(4) MR_TA_ST(5) MR_TA_ST(6) MR_TA_ST(7)
+                MR_TA_ST(8) MR_TA_ST(10)
+            default: break;
+            }
+        }
+#undef MR_TA_ST
+        Ns *= RR;
+    }
+}
+
+// FAST: a pencil's elements are contiguous (es = 1). LAST: store to `o`.
+template <bool FAST, bool LAST, int NT>
+__global__ void __launch_bounds__(NT, 4)
+mr_k_toep_axis(mr_fft_len<double> fn, mr_fft_len<double> fm, mr_ta_axis ax, mr_ta_out o,
+               const double *__restrict__ dc, long long npencil, int TX, mr_fdiv txdiv,
+               long long pbase)
+{
+    extern __shared__ __align__(16) unsigned char mr_smem[];
+    double2 *A = reinterpret_cast<double2 *>(mr_smem);
+    __shared__ long long base[MR_TA_MAXTX], cbase[MR_TA_MAXTX], comp[MR_TA_MAXTX];
+    __shared__ int cz[MR_TA_MAXTX];
+    const int nf = fn.n, M = fm.n, ns = mr_ta_at(nf) + 1;
+    const long long p0 = pbase + mr_xcd_block(blockIdx.x, gridDim.x) * TX;
+    const int tp = (int)((npencil - p0 < TX) ? (npencil - p0) : TX);
+    if (threadIdx.x < tp) {
+        const long long p = p0 + threadIdx.x;
+        const long long r = p / ax.n0, i = p - r * ax.n0;
+        const long long q = r / ax.n1, j = r - q * ax.n1;
+        base[threadIdx.x] = ax.s0 * i + ax.s1 * j + ax.s2 * q;
+        if (LAST) {
+            const long long qq = o.q0 + q;
+            cz[threadIdx.x] = (int)(qq % o.Nkz);
+            cbase[threadIdx.x] = i + o.c1 * j + (o.inv ? 0 : o.Ptr * qq);
+            comp[threadIdx.x] = qq / o.Nkz;
+        }
+    }
+    __syncthreads();
+    // all of a thread's loads before its LDS writes
+    double2 t[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int q = threadIdx.x + k * NT;
+        const int hi = (int)mr_fdiv_q(FAST ? fn.ndiv : txdiv, (unsigned)q);
+        const int lo = q - hi * (FAST ? nf : TX);
+        const int p = FAST ? hi : lo, e = FAST ? lo : hi;
+        const bool in = p < tp && e < nf;
+        t[k] = in ? ax.data[base[p] + (FAST ? e : ax.es * e)] : make_double2(0.0, 0.0);
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int q = threadIdx.x + k * NT;
+        const int hi = (int)mr_fdiv_q(FAST ? fn.ndiv : txdiv, (unsigned)q);
+        const int lo = q - hi * (FAST ? nf : TX);
+        const int p = FAST ? hi : lo, e = FAST ? lo : hi;
+        if (p < tp && e < nf) A[p * ns + mr_ta_at(e)] = t[k];
+    }
+    __syncthreads();
+    mr_ta_stages<false, false, NT>(A, fn, dc, nf, 0, fn.nst, ns, tp);
+    if (fm.nst > 0) mr_ta_stages<true, true, NT>(A, fm, dc, nf, 0, 1, ns, tp);
+    else mr_ta_stage<1, true, true, NT>(A, fm.tws, dc, nf, 1, ns, tp, 1, mr_fdiv{1, 0, 0},
+                                        mr_fdiv{1, 0, 0});
+    mr_ta_stages<true, false, NT>(A, fm, dc, nf, 1, fm.nst, ns, tp);
+    auto put = [&](int p, int e) {
+        int k = e + ax.shift;
+        if (k >= M) k -= M;
+        const double2 v = A[p * ns + mr_ta_at(e)];
+        if (!LAST) {
+            ax.data[base[p] + (FAST ? k : ax.es * k)] = v;
+            return;
+        }
+        const float2 w = make_float2((float)(v.x * o.scale), (float)(v.y * o.scale));
+        const long long c = cbase[p] + o.cs * k;
+        if (!o.inv) {
+            o.out[c] = w;
+        } else {
+            const int row = o.inv[c + o.Ptr * cz[p]];
+            if (row >= 0) o.out[row + o.nm * comp[p]] = w;
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int q = threadIdx.x + k * NT;
+        const int hi = (int)mr_fdiv_q(FAST ? fm.ndiv : txdiv, (unsigned)q);
+        const int lo = q - hi * (FAST ? M : TX);
+        const int p = FAST ? hi : lo, e = FAST ? lo : hi;
+        if (p < tp && e < M) put(p, e);
+    }
+}
+
 // inv[centered linear index] = mask row, -1 elsewhere
 __global__ void mr_k_mask_rows(int *inv, long long P, const int64_t *mask, long long nm)
 {
@@ -201,6 +409,75 @@ int mr_build_mask_rows(const mr_config *cfg, const int64_t *mask, hipStream_t s,
     return MR_SUCCESS;
 }
 
+// Every axis of qn fine grids in place, then the store of components q0 ...
+int mr_toep_axes(const toep_geom &tg, const mr_grid &g, double2 *fine, double *const *dc, int qn,
+                 long long q0, const int *inv, long long nm, float2 *out, hipStream_t s)
+{
+    const long long nx = g.nf[0], ny = g.nf[1], nz = g.nf[2];
+    const long long m0 = tg.M[0], m1 = tg.M[1];
+    for (int a = 0; a < tg.d; ++a) {
+        mr_fft_len<double> fn, fm;
+        MR_TRY(mr_fft_get<double>(g.nf[a], &fn));
+        MR_TRY(mr_fft_get<double>(tg.M[a], &fm));
+        mr_ta_axis ax{fine, 0, 0, 0, 0, 0, 1, tg.shift[a]};
+        long long np = 0;
+        if (a == 0) {
+            np = ny * nz * qn;
+            ax.n0 = np; ax.n1 = 1; ax.s0 = nx;
+        } else if (a == 1) {
+            np = m0 * nz * qn;
+            ax.n0 = m0; ax.n1 = nz; ax.s0 = 1; ax.s1 = nx * ny; ax.s2 = nx * ny * nz; ax.es = nx;
+        } else {
+            np = m0 * m1 * qn;
+            ax.n0 = m0; ax.n1 = m1; ax.s0 = 1; ax.s1 = nx; ax.s2 = nx * ny * nz; ax.es = nx * ny;
+        }
+        const mr_ta_out o{out, inv, m0, a == 2 ? m0 * m1 : m0, tg.Ptr, q0, nm, tg.Nkz, tg.scale};
+        const bool last = a == tg.d - 1;
+        // 8 NT values per workgroup: 256 threads where whole pencils fill them
+        // (more, smaller workgroups overlap their phases), else 512; along y
+        // and z 512 threads for wider rows
+        const int nf = g.nf[a];
+        const bool small = a == 0 && 2048 / nf * nf >= 1740;
+        const int NT = small ? 256 : 512;
+        int TX = 8 * NT / nf;
+        if (TX > MR_TA_MAXTX) TX = MR_TA_MAXTX;
+        if (a > 0) TX = mr_pow2_floor(TX);
+        const size_t lds = (size_t)TX * (mr_ta_at(nf) + 1) * sizeof(double2);
+        auto fn_k = a == 0 ? (small ? mr_k_toep_axis<true, false, 256>
+                                    : mr_k_toep_axis<true, false, 512>)
+                           : last ? mr_k_toep_axis<false, true, 512>
+                                  : mr_k_toep_axis<false, false, 512>;
+        if (lds > 65536)
+            MR_HIP_CHECK(hipFuncSetAttribute((const void *)fn_k,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        const long long blocks = mr_ceil_div(np, TX), maxb = mr_max_blocks(NT);
+        for (long long b0 = 0; b0 < blocks; b0 += maxb) {
+            const long long nb = blocks - b0 < maxb ? blocks - b0 : maxb;
+            hipLaunchKernelGGL(fn_k, dim3((unsigned)nb), dim3(NT), lds, s, fn, fm, ax, o, dc[a], np,
+                               TX, mr_fdiv_make((unsigned)TX), b0 * TX);
+            MR_LAUNCH_CHECK("mr_k_toep_axis");
+        }
+    }
+    return MR_SUCCESS;
+}
+
+// The same by separate passes, through the natural-order grids b.nat.
+int mr_toep_separate(const toep_geom &tg, const mr_grid &g, const toep_bufs &b, int qn,
+                     long long q0, long long nm, float2 *out, hipStream_t s)
+{
+    MR_TRY(mr_grid_fft(g, b.fine, nullptr, qn, false, s));
+    MR_GRID_CHECK(mr_ceil_div(tg.Ptr * qn, 256), 256, "mr_k_deconv");
+    hipLaunchKernelGGL(mr_k_deconv, dim3((unsigned)mr_ceil_div(tg.Ptr * qn, 256)), dim3(256), 0, s,
+                       b.fine, g, tg.Ptr, qn, b.dc[0], b.dc[1], b.dc[2], b.nat);
+    MR_LAUNCH_CHECK("mr_k_deconv");
+    MR_TRY(mr_toep_ifft(tg, b.nat, qn, s));
+    hipLaunchKernelGGL(mr_k_toep_store, dim3((unsigned)mr_ceil_div(tg.Ptr * qn, 256)), dim3(256), 0,
+                       s, b.nat, tg.M[0], tg.M[1], tg.M[2], tg.shift[0], tg.shift[1], tg.shift[2],
+                       tg.Ptr, qn, q0, tg.Nkz, tg.scale, b.inv, nm, out);
+    MR_LAUNCH_CHECK("mr_k_toep_store");
+    return MR_SUCCESS;
+}
+
 }  // namespace
 
 int mr_calc_toep_impl(const mr_config *cfg, const mr_complex *d_phi2, const float *d_traj,
@@ -236,10 +513,18 @@ int mr_calc_toep_impl(const mr_config *cfg, const mr_complex *d_phi2, const floa
     }
     if (cfg->is_masked) MR_TRY(mr_build_mask_rows(cfg, d_mask, s, &b.inv));
 
-    // Chunk of components: fine grids + natural-order grids within budget.
+    // the one-pass axes need unrolled butterflies for the mode counts (the
+    // fine counts always have them)
+    bool onepass = true;
+    for (int a = 0; a < tg.d; ++a)
+        onepass = onepass && mr_fft_smooth(tg.M[a]) && g.nf[a] <= 4096;
+
+    // Chunk of components: fine grids (and natural-order grids for the
+    // separate passes) within budget.
     size_t budget = 0;
     MR_TRY(mr_mem_budget(cfg, &budget));
-    const size_t per_q = ((size_t)g.nfine + (size_t)tg.Ptr + (size_t)smp.part_elems(1)) * sizeof(double2);
+    const size_t per_q = ((size_t)g.nfine + (onepass ? 0 : (size_t)tg.Ptr) +
+                          (size_t)smp.part_elems(1)) * sizeof(double2);
     long long Qc = (long long)(budget / 2 / per_q);
     const long long cap = mr_env_ll("MR_AHA_TOEP_MAX_CHUNK", 0);
     if (cap > 0 && Qc > cap) Qc = cap;
@@ -247,7 +532,8 @@ int mr_calc_toep_impl(const mr_config *cfg, const mr_complex *d_phi2, const floa
     if (Qc > 65535LL * 16) Qc = 65535LL * 16;
     if (Qc < 1) Qc = 1;
     hipError_t e = hipMalloc((void **)&b.fine, (size_t)g.nfine * Qc * sizeof(double2));
-    if (e == hipSuccess) e = hipMalloc((void **)&b.nat, (size_t)tg.Ptr * Qc * sizeof(double2));
+    if (e == hipSuccess && !onepass)
+        e = hipMalloc((void **)&b.nat, (size_t)tg.Ptr * Qc * sizeof(double2));
     if (e == hipSuccess && smp.next > 0)
         e = hipMalloc((void **)&b.part, (size_t)smp.part_elems(Qc) * sizeof(double2));
     if (e != hipSuccess) {
@@ -260,17 +546,12 @@ int mr_calc_toep_impl(const mr_config *cfg, const mr_complex *d_phi2, const floa
     for (long long q0 = 0; q0 < Q; q0 += Qc) {
         const int qn = (int)((Q - q0 < Qc) ? Q - q0 : Qc);
         MR_TRY(mr_grid_spread(g, smp, b.c, (int)Q, (int)q0, qn, b.fine, b.part, s));
-        MR_TRY(mr_grid_fft(g, b.fine, nullptr, qn, false, s));
-        MR_GRID_CHECK(mr_ceil_div(tg.Ptr * qn, 256), 256, "mr_k_deconv");
-        hipLaunchKernelGGL(mr_k_deconv, dim3((unsigned)mr_ceil_div(tg.Ptr * qn, 256)), dim3(256),
-                           0, s, b.fine, g, tg.Ptr, qn, b.dc[0], b.dc[1], b.dc[2], b.nat);
-        MR_LAUNCH_CHECK("mr_k_deconv");
-        MR_TRY(mr_toep_ifft(tg, b.nat, qn, s));
-        hipLaunchKernelGGL(mr_k_toep_store, dim3((unsigned)mr_ceil_div(tg.Ptr * qn, 256)),
-                           dim3(256), 0, s, b.nat, tg.M[0], tg.M[1], tg.M[2], tg.shift[0],
-                           tg.shift[1], tg.shift[2], tg.Ptr, qn, q0, tg.Nkz, tg.scale, b.inv,
-                           (long long)cfg->num_masked, reinterpret_cast<float2 *>(d_out));
-        MR_LAUNCH_CHECK("mr_k_toep_store");
+        if (onepass)
+            MR_TRY(mr_toep_axes(tg, g, b.fine, b.dc, qn, q0, b.inv, (long long)cfg->num_masked,
+                                reinterpret_cast<float2 *>(d_out), s));
+        else
+            MR_TRY(mr_toep_separate(tg, g, b, qn, q0, (long long)cfg->num_masked,
+                                    reinterpret_cast<float2 *>(d_out), s));
         if (cfg->verbose)
             printf("[mr_aha] calc_toep: components %lld-%lld of %lld issued\n", q0, q0 + qn - 1, Q);
     }

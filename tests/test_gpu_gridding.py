@@ -94,3 +94,33 @@ def test_nufft_tiles(mr, tt, n, L, spokes, nkx):
     with mr.create_op(cfg, dev(S), dev(phi2), dev(traj), method="nufft") as op:
         y = op(dev(x)).cpu().numpy()
     assert rel(y, nudft.aha_nudft(g, x, S, phi2, traj)) < 1e-5 + 2e-7
+
+
+# mode counts that start with every radix (14 = 2 7, 9 = 3 3, 12 = 6 2, ...), a
+# single mode, pencils of several workgroups and a partial last one, and
+# counts without an unrolled butterfly (22, 13: the separate passes)
+AXES = [("2D", (8, 7), (16, 14)), ("2D", (5, 6), (9, 12)), ("2D", (9, 9), (25, 35)),
+        ("2D", (1, 20), (1, 40)), ("2D", (130, 4), (260, 8)), ("2D", (11, 6), (22, 13)),
+        ("2D", (4, 96), (8, 192)), ("stack", (18, 12, 3), (36, 24, 3)),
+        ("3D", (5, 4, 7), (10, 8, 14)), ("3D", (6, 3, 9), (12, 7, 18)), ("3D", (4, 5, 3), (8, 11, 6))]
+
+
+@pytest.mark.parametrize("tt,n,M", AXES)
+@pytest.mark.parametrize("chunk", [0, 2])
+def test_kernel_build_axes(mr, tt, n, M, chunk, monkeypatch):
+    from oracle import conventions as cv
+    from oracle import toeplitz
+    print(f"[gridding] axes {tt} {n} grid {M} chunk={chunk}", flush=True)
+    if chunk:
+        monkeypatch.setenv("MR_AHA_TOEP_MAX_CHUNK", str(chunk))
+        monkeypatch.setenv("MR_AHA_HIP_MAX_BLOCKS", "7")
+    L = 2
+    _, traj, phi2 = _problem(tt, n, L, 20, 16, 3)
+    g = cv.make_geometry(tt, n, L, 1, M)
+    cfg = mr.make_config(tt, n, L, phi2_dim=M)
+    K = mr.calc_toep(cfg, dev(phi2), dev(traj))
+    assert rel(K.cpu().numpy(), toeplitz.calc_kernel(g, phi2, traj)) < 1e-5
+    mask = torch.arange(0, int(np.prod(M)), 3, device="cuda")
+    cfgm = mr.make_config(tt, n, L, phi2_dim=M, is_masked=True, num_masked=mask.numel())
+    Km = mr.calc_toep(cfgm, dev(phi2), dev(traj), mask)
+    assert torch.equal(torch.view_as_real(Km), torch.view_as_real(K.reshape(K.shape[0], -1)[:, mask]))
