@@ -643,6 +643,9 @@ int mr_mem_budget(const mr_config *cfg, size_t *budget)
 {
     size_t fr = 0, tot = 0;
     MR_HIP_CHECK(hipMemGetInfo(&fr, &tot));
+    int dev = 0;
+    MR_HIP_CHECK(hipGetDevice(&dev));
+    fr += mr_ws_idle_bytes(dev);
     double f = cfg->mem_fraction;
     if (!(f > 0.0)) f = 0.5;
     if (f > 0.95) f = 0.95;
@@ -818,9 +821,9 @@ static int mr_plan_create_impl(const mr_config *cfg, mr_aha_plan *out)
         const size_t abytes = a_per * group * sizeof(float2);
         const size_t bbytes = b_per * group * sizeof(float2);
         hipError_t e = hipSuccess;
-        if (abytes) e = hipMalloc((void **)&p->bufA, abytes);
-        if (e == hipSuccess) e = hipMalloc((void **)&p->bufB, bbytes);
-        if (e == hipSuccess && inv_bytes) e = hipMalloc((void **)&p->d_inv, inv_bytes);
+        if (abytes) e = mr_dev_malloc((void **)&p->bufA, abytes);
+        if (e == hipSuccess) e = mr_dev_malloc((void **)&p->bufB, bbytes);
+        if (e == hipSuccess && inv_bytes) e = mr_dev_malloc((void **)&p->d_inv, inv_bytes);
         if (e == hipSuccess) break;
         (void)hipGetLastError();
         mr_plan_free_buffers(p);

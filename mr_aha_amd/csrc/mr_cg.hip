@@ -448,11 +448,11 @@ extern "C" MR_EXPORT int mr_op_cg(mr_op op, mr_op op_refresh, const mr_complex *
     cg_ws w;
     int rc = MR_SUCCESS;
     const size_t vb = (size_t)n * sizeof(float2);
-    if (hipMalloc((void **)&w.r, vb) != hipSuccess || hipMalloc((void **)&w.p, vb) != hipSuccess ||
-        hipMalloc((void **)&w.Ap, vb) != hipSuccess ||
-        hipMalloc((void **)&w.part, CG_BLOCKS * sizeof(double2)) != hipSuccess ||
-        hipMalloc((void **)&w.scal, S_N * sizeof(double)) != hipSuccess ||
-        hipMalloc((void **)&w.hist, (size_t)(n_iter + 2) * sizeof(double)) != hipSuccess) {
+    if (mr_dev_malloc((void **)&w.r, vb) != hipSuccess || mr_dev_malloc((void **)&w.p, vb) != hipSuccess ||
+        mr_dev_malloc((void **)&w.Ap, vb) != hipSuccess ||
+        mr_dev_malloc((void **)&w.part, CG_BLOCKS * sizeof(double2)) != hipSuccess ||
+        mr_dev_malloc((void **)&w.scal, S_N * sizeof(double)) != hipSuccess ||
+        mr_dev_malloc((void **)&w.hist, (size_t)(n_iter + 2) * sizeof(double)) != hipSuccess) {
         (void)hipGetLastError();
         mr_set_error("mr_op_cg: failed to allocate %zu bytes of work vectors", 3 * vb);
         rc = MR_ERR_ALLOC;

@@ -37,13 +37,22 @@ void mr_grid_setup(mr_grid *g, int d, const int *M, double eps)
     }
 }
 
-// Gauss-Legendre nodes/weights on [-1, 1] by Newton iteration on P_n.
-static void mr_gauss_legendre(int n, std::vector<double> &x, std::vector<double> &wq)
+namespace {
+
+// Quadrature of the kernel's transform: Gauss-Legendre nodes on [-1, 1] and
+// their weights times the kernel's value there (2 w + 60 nodes).
+struct mr_grid_quad {
+    int n;
+    double z[2 * MR_GRID_MAXW + 60], f[2 * MR_GRID_MAXW + 60];
+};
+
+// Newton iteration on P_n for the nodes z > 0 (the others mirror them).
+mr_grid_quad mr_make_quad(int w, double beta)
 {
-    x.resize(n);
-    wq.resize(n);
-    for (int i = 0; i < n; ++i) {
-        double z = std::cos(M_PI * (i + 0.75) / (n + 0.5));
+    mr_grid_quad q;
+    const int n = q.n = 2 * w + 60;   // even
+    for (int i = 0; i < n / 2; ++i) {
+        double z = std::cos(M_PI * (i + 0.75) / (n + 0.5)), dp = 1.0;
         for (int it = 0; it < 100; ++it) {
             double p0 = 1.0, p1 = z;
             for (int k = 2; k <= n; ++k) {
@@ -51,42 +60,43 @@ static void mr_gauss_legendre(int n, std::vector<double> &x, std::vector<double>
                 p0 = p1;
                 p1 = p2;
             }
-            const double dp = n * (z * p1 - p0) / (z * z - 1.0);
+            dp = n * (z * p1 - p0) / (z * z - 1.0);
             const double dz = p1 / dp;
             z -= dz;
-            if (std::fabs(dz) < 1e-16) break;
+            if (std::fabs(dz) < 1e-15) break;
         }
-        double p0 = 1.0, p1 = z;
-        for (int k = 2; k <= n; ++k) {
-            const double p2 = ((2.0 * k - 1.0) * z * p1 - (k - 1.0) * p0) / k;
-            p0 = p1;
-            p1 = p2;
-        }
-        const double dp = n * (z * p1 - p0) / (z * z - 1.0);
-        x[i] = z;
-        wq[i] = 2.0 / ((1.0 - z * z) * dp * dp);
+        const double wq = 2.0 / ((1.0 - z * z) * dp * dp);
+        q.z[i] = z;
+        q.z[n - 1 - i] = -z;
+        q.f[i] = q.f[n - 1 - i] = wq * std::exp(beta * (std::sqrt(1.0 - z * z) - 1.0));
     }
+    return q;
 }
 
-std::vector<double> mr_grid_deconv(const mr_grid &g, int a)
+}  // namespace
+
+// Deconvolution factors 1/phi_hat(delta) of one axis, natural order.
+__global__ void mr_k_grid_deconv(mr_grid_quad q, int M, int nf, int w, double *dc)
 {
-    const int M = g.M[a];
-    std::vector<double> out(M, 1.0);
-    if (a >= g.d) return out;
-    std::vector<double> zq, wq;
-    mr_gauss_legendre(2 * g.w + 60, zq, wq);
-    const int nf = g.nf[a];
-    const int half = M / 2;
-    for (int j = 0; j < M; ++j) {
-        const int delta = (j < M - half) ? j : j - M;
-        double s = 0.0;
-        for (size_t i = 0; i < zq.size(); ++i) {
-            const double phi = std::exp(g.beta * (std::sqrt(1.0 - zq[i] * zq[i]) - 1.0));
-            s += wq[i] * phi * std::cos(delta * M_PI * g.w * zq[i] / nf);
-        }
-        out[j] = 1.0 / (0.5 * g.w * s);
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= M) return;
+    const int delta = (j < M - M / 2) ? j : j - M;
+    const double c = (double)delta * w / nf;
+    double s = 0.0;
+    for (int i = 0; i < q.n; ++i) s += q.f[i] * cospi(c * q.z[i]);
+    dc[j] = 1.0 / (0.5 * w * s);
+}
+
+int mr_grid_deconv(const mr_grid &g, double **dc, hipStream_t stream)
+{
+    const mr_grid_quad q = mr_make_quad(g.w, g.beta);
+    for (int a = 0; a < g.d; ++a) {
+        MR_HIP_CHECK(mr_dev_malloc((void **)&dc[a], g.M[a] * sizeof(double)));
+        hipLaunchKernelGGL(mr_k_grid_deconv, dim3((unsigned)mr_ceil_div(g.M[a], 64)), dim3(64), 0,
+                           stream, q, g.M[a], g.nf[a], g.w, dc[a]);
+        MR_LAUNCH_CHECK("mr_k_grid_deconv");
     }
-    return out;
+    return MR_SUCCESS;
 }
 
 __device__ __forceinline__ double mr_es(double z, double beta)
@@ -227,13 +237,11 @@ __global__ void mr_k_grid_ext_list(long long nbins, const int *ext, const int *b
     for (int k = 0; k < ext[tile]; ++k) list[base[tile] + k] = make_int2((int)tile, k + 1);
 }
 
-void mr_grid_samples_free(mr_grid_samples *s)
+void mr_grid_samples_free(mr_grid_samples *s, bool idle)
 {
-    if (s->i0) (void)hipFree(s->i0);
-    if (s->rd) (void)hipFree(s->rd);
-    if (s->wt) (void)hipFree(s->wt);
-    if (s->start) (void)hipFree(s->start);
-    if (s->ext) (void)hipFree(s->ext);
+    if (!idle) (void)hipDeviceSynchronize();
+    void *bufs[] = {s->i0, s->rd, s->wt, s->start, s->ext};
+    for (void *p : bufs) mr_ws_put(p);
     *s = mr_grid_samples();
 }
 
@@ -252,7 +260,9 @@ int mr_grid_samples_build(const mr_grid &g, const float *traj, long long Ntrajs,
     hipError_t e = hipSuccess;
     int end_bit = 1;
     while (end_bit < 32 && (g.nbins >> end_bit) != 0) ++end_bit;
-#define MR_GA(ptr, bytes) if (e == hipSuccess) e = hipMalloc((void **)&(ptr), (bytes))
+#define MR_GA(ptr, bytes)                                                       \
+    if (e == hipSuccess && !((ptr) = (decltype(ptr))mr_ws_get(bytes)))         \
+        e = hipErrorOutOfMemory
     MR_GA(keys, n * sizeof(unsigned));
     MR_GA(keys2, n * sizeof(unsigned));
     MR_GA(vals, n * sizeof(int));
@@ -305,7 +315,8 @@ int mr_grid_samples_build(const mr_grid &g, const float *traj, long long Ntrajs,
         if (e == hipSuccess) e = hipStreamSynchronize(stream);
         if (e == hipSuccess && total > 0) {
             s.next = total;
-            e = hipMalloc((void **)&s.ext, (size_t)total * sizeof(int2));
+            s.ext = (int2 *)mr_ws_get((size_t)total * sizeof(int2));
+            if (!s.ext) e = hipErrorOutOfMemory;
             if (e == hipSuccess) {
                 hipLaunchKernelGGL(mr_k_grid_ext_list, dim3(bblk), dim3(256), 0, stream, g.nbins,
                                    ext, base, s.ext);
@@ -319,10 +330,11 @@ int mr_grid_samples_build(const mr_grid &g, const float *traj, long long Ntrajs,
             rc = MR_ERR_CUFINUFFT;
         }
     }
+    if (rc != MR_SUCCESS) (void)hipStreamSynchronize(stream);   // nothing in flight
     void *scratch[] = {tmp, keys, keys2, vals, perm, ext, base};
-    for (void *p : scratch) if (p) (void)hipFree(p);
+    for (void *p : scratch) mr_ws_put(p);
     if (rc != MR_SUCCESS) {
-        mr_grid_samples_free(&s);
+        mr_grid_samples_free(&s, true);
         return rc;
     }
     *out = s;

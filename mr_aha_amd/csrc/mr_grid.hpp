@@ -13,8 +13,6 @@
 
 #include "mr_hip.hpp"
 
-#include <vector>
-
 #define MR_GRID_MAXW 16
 
 struct mr_grid {
@@ -32,9 +30,11 @@ struct mr_grid {
 // Fill the geometry for `d` transformed axes with mode counts M[0..d-1].
 void mr_grid_setup(mr_grid *g, int d, const int *M, double eps);
 
-// Deconvolution factors 1/phi_hat(delta) for the modes of axis a in
-// natural order (index j <-> delta = j or j - M). Host vector.
-std::vector<double> mr_grid_deconv(const mr_grid &g, int a);
+// Deconvolution factors 1/phi_hat(delta) of the modes of every transformed
+// axis a < d in natural order (index j <-> delta = j or j - M), into dc[a]
+// allocated here (the caller frees it), on `stream`. dc[a] of the other axes
+// stays as it is: their only mode has factor one.
+int mr_grid_deconv(const mr_grid &g, double **dc, hipStream_t stream);
 
 // Candidate samples per segment of mr_k_spread: a wavefront's share of a tile.
 // Large enough that few tiles are split (each extra segment costs a partial
@@ -64,7 +64,9 @@ struct mr_grid_samples {
 // (first `g.d` coordinates used) on `stream`. Synchronous.
 int mr_grid_samples_build(const mr_grid &g, const float *traj, long long Ntrajs, long long Nkx,
                           hipStream_t stream, mr_grid_samples *out);
-void mr_grid_samples_free(mr_grid_samples *s);
+// Give the tables back to the kept scratch; unless `idle` (no work that uses
+// them is pending) the device is waited for first, as hipFree would.
+void mr_grid_samples_free(mr_grid_samples *s, bool idle);
 
 // Type-1 spreading of Q strength sets (strength of a sample of readout s, set
 // q: str[s * qs + q0 + q], i.e. constant along a readout) onto Q fine

@@ -66,9 +66,9 @@ static int mr_calc_mask_impl(const mr_config *cfg, const float *d_traj, int64_t 
     void *tmp = nullptr;
     size_t tmp_bytes = 0;
     int rc = MR_SUCCESS;
-    hipError_t e = hipMalloc((void **)&a, n);
-    if (e == hipSuccess) e = hipMalloc((void **)&b, n);
-    if (e == hipSuccess) e = hipMalloc((void **)&d_cnt, sizeof(int64_t));
+    hipError_t e = mr_dev_malloc((void **)&a, n);
+    if (e == hipSuccess) e = mr_dev_malloc((void **)&b, n);
+    if (e == hipSuccess) e = mr_dev_malloc((void **)&d_cnt, sizeof(int64_t));
     if (e != hipSuccess) {
         (void)hipGetLastError();
         rc = MR_ERR_ALLOC;
@@ -96,12 +96,12 @@ static int mr_calc_mask_impl(const mr_config *cfg, const float *d_traj, int64_t 
         int64_t *dst = d_mask;
         int64_t *scratch_out = nullptr;
         if (e == hipSuccess && !dst) {
-            e = hipMalloc((void **)&scratch_out, n * sizeof(int64_t));
+            e = mr_dev_malloc((void **)&scratch_out, n * sizeof(int64_t));
             dst = scratch_out;
         }
         if (e == hipSuccess)
             e = hipcub::DeviceSelect::Flagged(nullptr, tmp_bytes, first, a, dst, d_cnt, (int64_t)n, s);
-        if (e == hipSuccess) e = hipMalloc(&tmp, tmp_bytes ? tmp_bytes : 1);
+        if (e == hipSuccess) e = mr_dev_malloc(&tmp, tmp_bytes ? tmp_bytes : 1);
         if (e == hipSuccess)
             e = hipcub::DeviceSelect::Flagged(tmp, tmp_bytes, first, a, dst, d_cnt, (int64_t)n, s);
         int64_t kept = 0;

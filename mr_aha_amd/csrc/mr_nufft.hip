@@ -13,7 +13,6 @@
 #include "mr_grid.hpp"
 
 #include <new>
-#include <vector>
 
 struct mr_nufft_eng {
     mr_config cfg;
@@ -38,7 +37,7 @@ struct mr_nufft_eng {
 
 static void mr_nufft_free(mr_nufft_eng *e)
 {
-    mr_grid_samples_free(&e->smp);
+    mr_grid_samples_free(&e->smp, false);
     for (double *p : e->dc) if (p) (void)hipFree(p);
     void *bufs[] = {e->phi2, e->img, e->acc, e->fine, e->k1, e->k2, e->part};
     for (void *p : bufs) if (p) (void)hipFree(p);
@@ -75,25 +74,19 @@ int mr_nufft_eng_create(const mr_config *cfg, const mr_complex *d_phi2, const fl
     if (rc != MR_SUCCESS) { mr_nufft_free(e); return rc; }
     const size_t phi2_bytes = (size_t)Ntrajs * e->Nkz * cfg->L * cfg->L * sizeof(float2);
     const size_t img_bytes = (size_t)e->Nimg * cfg->L * sizeof(double2);
-    hipError_t he = hipMalloc((void **)&e->phi2, phi2_bytes);
-    if (he == hipSuccess) he = hipMalloc((void **)&e->img, img_bytes);
-    if (he == hipSuccess) he = hipMalloc((void **)&e->acc, img_bytes);
-    if (he == hipSuccess) he = hipMalloc((void **)&e->fine, (size_t)e->Q * e->g.nfine * sizeof(double2));
-    if (he == hipSuccess) he = hipMalloc((void **)&e->k1, (size_t)e->Q * e->Mnu * sizeof(double2));
+    hipError_t he = mr_dev_malloc((void **)&e->phi2, phi2_bytes);
+    if (he == hipSuccess) he = mr_dev_malloc((void **)&e->img, img_bytes);
+    if (he == hipSuccess) he = mr_dev_malloc((void **)&e->acc, img_bytes);
+    if (he == hipSuccess) he = mr_dev_malloc((void **)&e->fine, (size_t)e->Q * e->g.nfine * sizeof(double2));
+    if (he == hipSuccess) he = mr_dev_malloc((void **)&e->k1, (size_t)e->Q * e->Mnu * sizeof(double2));
     if (he == hipSuccess)
-        he = hipMalloc((void **)&e->k2,
+        he = mr_dev_malloc((void **)&e->k2,
                        ((size_t)e->Q * e->Mnu + MR_GRID_STR_PAD) * sizeof(double2));
     if (he == hipSuccess && e->smp.next > 0)
-        he = hipMalloc((void **)&e->part, (size_t)e->smp.part_elems(e->Q) * sizeof(double2));
-    for (int a = 0; a < 3 && he == hipSuccess; ++a) {
-        std::vector<double> dc = mr_grid_deconv(e->g, a);
-        he = hipMalloc((void **)&e->dc[a], dc.size() * sizeof(double));
-        // stream-ordered (never the legacy stream, which could tie this call
-        // to another thread's graph capture); synchronised below
-        if (he == hipSuccess)
-            he = hipMemcpyAsync(e->dc[a], dc.data(), dc.size() * sizeof(double),
-                                hipMemcpyHostToDevice, e->s);
-        if (he == hipSuccess) he = hipStreamSynchronize(e->s);
+        he = mr_dev_malloc((void **)&e->part, (size_t)e->smp.part_elems(e->Q) * sizeof(double2));
+    if (he == hipSuccess) {
+        rc = mr_grid_deconv(e->g, e->dc, e->s);
+        if (rc != MR_SUCCESS) { mr_nufft_free(e); return rc; }
     }
     if (he == hipSuccess)
         he = hipMemcpyAsync(e->phi2, d_phi2, phi2_bytes, hipMemcpyDeviceToDevice, e->s);
@@ -158,7 +151,7 @@ __global__ void mr_k_nu_pad(const double2 *img, mr_grid g, long long Nplane, int
         const int iimg = r + N / 2;       // image index
         int jn = r; if (jn < 0) jn += N;  // natural mode index
         const double *dc = (a == 0) ? dc0 : (a == 1) ? dc1 : dc2;
-        w *= dc[jn];
+        if (a < g.d) w *= dc[jn];
         src += mul * iimg;
         mul *= N;
     }
@@ -186,7 +179,7 @@ __global__ void mr_k_nu_crop(const double2 *fine, mr_grid g, long long Nplane, i
         int jn = r; if (jn < 0) jn += N;
         int f = r; if (f < 0) f += nf;
         const double *dc = (a == 0) ? dc0 : (a == 1) ? dc1 : dc2;
-        w *= dc[jn];
+        if (a < g.d) w *= dc[jn];
         fl += mul * f;
         mul *= nf;
     }

@@ -186,8 +186,8 @@ static int mr_op_create_impl(const mr_config *cfg, const mr_op_inputs *in,
         p->d_SEs = in->d_SEs;
         p->d_mask = mask_bytes ? in->d_mask : nullptr;
     } else {
-        hipError_t e = hipMalloc((void **)&p->own_SEs, se_bytes);
-        if (e == hipSuccess && mask_bytes) e = hipMalloc((void **)&p->own_mask, mask_bytes);
+        hipError_t e = mr_dev_malloc((void **)&p->own_SEs, se_bytes);
+        if (e == hipSuccess && mask_bytes) e = mr_dev_malloc((void **)&p->own_mask, mask_bytes);
         if (e == hipSuccess)
             e = hipMemcpyAsync(p->own_SEs, in->d_SEs, se_bytes, hipMemcpyDeviceToDevice, p->stream);
         if (e == hipSuccess && mask_bytes)
@@ -208,7 +208,7 @@ static int mr_op_create_impl(const mr_config *cfg, const mr_op_inputs *in,
             if (share) {
                 p->d_toep = in->d_phi2_toep;
             } else {
-                hipError_t e = hipMalloc((void **)&p->own_toep, toep_bytes);
+                hipError_t e = mr_dev_malloc((void **)&p->own_toep, toep_bytes);
                 if (e == hipSuccess)
                     e = hipMemcpyAsync(p->own_toep, in->d_phi2_toep, toep_bytes,
                                        hipMemcpyDeviceToDevice, p->stream);
@@ -223,7 +223,7 @@ static int mr_op_create_impl(const mr_config *cfg, const mr_op_inputs *in,
             }
         } else {
             const auto t0 = std::chrono::steady_clock::now();
-            if (hipMalloc((void **)&p->own_toep, toep_bytes) != hipSuccess) {
+            if (mr_dev_malloc((void **)&p->own_toep, toep_bytes) != hipSuccess) {
                 (void)hipGetLastError();
                 mr_op_release(p);
                 MR_FAIL(MR_ERR_ALLOC, "device %d: failed to allocate the %.2f GB copy of phi2_toep",
@@ -402,8 +402,8 @@ extern "C" MR_EXPORT int mr_op_set_kernel_format(mr_op op, int format)
             const int L = op->cfg.L;
             const long long T = (long long)L * (L + 1) / 2;
             const long long NB = (long long)((L + 3) / 4) * ((L + 3) / 4 + 1) / 2;
-            if (hipMalloc((void **)&q, (size_t)(T * kcol) * 4) != hipSuccess ||
-                hipMalloc((void **)&sc, (size_t)(NB * kcol) * 4) != hipSuccess) {
+            if (mr_dev_malloc((void **)&q, (size_t)(T * kcol) * 4) != hipSuccess ||
+                mr_dev_malloc((void **)&sc, (size_t)(NB * kcol) * 4) != hipSuccess) {
                 (void)hipGetLastError();
                 mr_set_error("mr_op_set_kernel_format: failed to allocate the 16-bit kernel "
                              "(%lld bytes)", (T + NB) * kcol * 4);

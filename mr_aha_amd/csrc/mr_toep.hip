@@ -72,7 +72,7 @@ __global__ void mr_k_deconv(const double2 *fine, mr_grid g, long long Ptr, int Q
         f[a] = dlt;
     }
     const long long fl = f[0] + (long long)g.nf[0] * (f[1] + (long long)g.nf[1] * f[2]);
-    const double s = dc0[jx] * dc1[jy] * dc2[jz];
+    const double s = dc0[jx] * dc1[jy] * (dc2 ? dc2[jz] : 1.0);
     const double2 v = fine[fl + g.nfine * q];
     nat[id] = make_double2(v.x * s, v.y * s);
 }
@@ -336,6 +336,9 @@ __global__ void mr_k_fill_i32(int *p, long long n, int v)
     if (i < n) p[i] = v;
 }
 
+// Bytes of gridding scratch a build aims at per chunk of components.
+#define MR_TOEP_CHUNK_BYTES (2LL << 30)
+
 namespace {
 
 struct toep_geom {
@@ -381,25 +384,32 @@ int mr_toep_ifft(const toep_geom &tg, double2 *nat, int Qc, hipStream_t s)
     return MR_SUCCESS;
 }
 
+// Scratch of one call; its work on `s` has ended, or is waited for, before
+// the blocks go back.
 struct toep_bufs {
+    hipStream_t s;
+    bool done = false;
+    mr_grid_samples smp;
     double2 *c = nullptr, *fine = nullptr, *nat = nullptr, *part = nullptr;
     double *dc[3] = {nullptr, nullptr, nullptr};
     int *inv = nullptr;
+    explicit toep_bufs(hipStream_t st) : s(st) {}
+    toep_bufs(const toep_bufs &) = delete;
     ~toep_bufs()
     {
-        if (c) (void)hipFree(c);
-        if (fine) (void)hipFree(fine);
-        if (nat) (void)hipFree(nat);
-        if (part) (void)hipFree(part);
+        if (!done) (void)hipStreamSynchronize(s);
+        void *bufs[] = {c, fine, nat, part, inv};
+        for (void *p : bufs) mr_ws_put(p);
         for (double *p : dc) if (p) (void)hipFree(p);
-        if (inv) (void)hipFree(inv);
+        mr_grid_samples_free(&smp, true);
     }
 };
 
 int mr_build_mask_rows(const mr_config *cfg, const int64_t *mask, hipStream_t s, int **inv)
 {
     const long long P = mr_pad_size(cfg), nm = cfg->num_masked;
-    MR_HIP_CHECK(hipMalloc((void **)inv, P * sizeof(int)));
+    *inv = (int *)mr_ws_get(P * sizeof(int));
+    if (!*inv) MR_FAIL(MR_ERR_ALLOC, "failed to allocate the mask rows of %lld locations", P);
     hipLaunchKernelGGL(mr_k_fill_i32, dim3((unsigned)mr_ceil_div(P, 256)), dim3(256), 0, s, *inv,
                        P, -1);
     MR_LAUNCH_CHECK("mr_k_fill_i32");
@@ -490,27 +500,17 @@ int mr_calc_toep_impl(const mr_config *cfg, const mr_complex *d_phi2, const floa
 
     mr_grid g;
     mr_grid_setup(&g, tg.d, tg.M, cfg->eps);
-    toep_bufs b;
-    mr_grid_samples smp;
+    toep_bufs b(s);
+    mr_grid_samples &smp = b.smp;
     MR_TRY(mr_grid_samples_build(g, d_traj, Ntrajs, Nkx, s, &smp));
-    struct samples_guard {
-        mr_grid_samples *p;
-        ~samples_guard() { mr_grid_samples_free(p); }
-    } guard{&smp};
 
-    MR_HIP_CHECK(hipMalloc((void **)&b.c, (Q * Ntrajs + MR_GRID_STR_PAD) * sizeof(double2)));
+    b.c = (double2 *)mr_ws_get((Q * Ntrajs + MR_GRID_STR_PAD) * sizeof(double2));
+    if (!b.c) MR_FAIL(MR_ERR_ALLOC, "failed to allocate the strengths of %lld components", Q);
     hipLaunchKernelGGL(mr_k_pack_strengths, dim3((unsigned)mr_ceil_div(Q * Ntrajs, 256)),
                        dim3(256), 0, s, reinterpret_cast<const float2 *>(d_phi2), (long long)Ntrajs,
                        tg.Nkz, cfg->L, cfg->triangulation == MR_TRI_UPPER ? 1 : 0, T, b.c);
     MR_LAUNCH_CHECK("mr_k_pack_strengths");
-    for (int a = 0; a < 3; ++a) {
-        std::vector<double> dc = mr_grid_deconv(g, a);
-        MR_HIP_CHECK(hipMalloc((void **)&b.dc[a], dc.size() * sizeof(double)));
-        // stream-ordered, not on the legacy stream (see mr_fft_get)
-        MR_HIP_CHECK(hipMemcpyAsync(b.dc[a], dc.data(), dc.size() * sizeof(double),
-                                    hipMemcpyHostToDevice, s));
-        MR_HIP_CHECK(hipStreamSynchronize(s));
-    }
+    MR_TRY(mr_grid_deconv(g, b.dc, s));
     if (cfg->is_masked) MR_TRY(mr_build_mask_rows(cfg, d_mask, s, &b.inv));
 
     // the one-pass axes need unrolled butterflies for the mode counts (the
@@ -526,17 +526,24 @@ int mr_calc_toep_impl(const mr_config *cfg, const mr_complex *d_phi2, const floa
     const size_t per_q = ((size_t)g.nfine + (onepass ? 0 : (size_t)tg.Ptr) +
                           (size_t)smp.part_elems(1)) * sizeof(double2);
     long long Qc = (long long)(budget / 2 / per_q);
+    // A chunk beyond a few GB gains nothing (192x192x32 L=8: 15.2 ms with 1.2 GB
+    // chunks, 15.4 with all 10.9 GB), and giving that much memory back stalls
+    // the call now and then (250 ms for 9 GB and more). Below four components a
+    // spread has too few strengths for the weights it forms (96^3 L=4, 0.9 GB
+    // each: 28 ms one at a time, 22.5 in twos, 19.4 in fours).
+    long long fit = (long long)(MR_TOEP_CHUNK_BYTES / per_q);
+    if (fit < 4) fit = 4;
+    if (Qc > fit) Qc = mr_ceil_div(Q, mr_ceil_div(Q, fit));   // even chunks
     const long long cap = mr_env_ll("MR_AHA_TOEP_MAX_CHUNK", 0);
     if (cap > 0 && Qc > cap) Qc = cap;
     if (Qc > Q) Qc = Q;
     if (Qc > 65535LL * 16) Qc = 65535LL * 16;
     if (Qc < 1) Qc = 1;
-    hipError_t e = hipMalloc((void **)&b.fine, (size_t)g.nfine * Qc * sizeof(double2));
-    if (e == hipSuccess && !onepass)
-        e = hipMalloc((void **)&b.nat, (size_t)tg.Ptr * Qc * sizeof(double2));
-    if (e == hipSuccess && smp.next > 0)
-        e = hipMalloc((void **)&b.part, (size_t)smp.part_elems(Qc) * sizeof(double2));
-    if (e != hipSuccess) {
+    b.fine = (double2 *)mr_ws_get((size_t)g.nfine * Qc * sizeof(double2));
+    if (!onepass) b.nat = (double2 *)mr_ws_get((size_t)tg.Ptr * Qc * sizeof(double2));
+    if (smp.next > 0)
+        b.part = (double2 *)mr_ws_get((size_t)smp.part_elems(Qc) * sizeof(double2));
+    if (!b.fine || (!onepass && !b.nat) || (smp.next > 0 && !b.part)) {
         (void)hipGetLastError();
         MR_FAIL(MR_ERR_ALLOC,
                 "failed to allocate the calc_toep chunk buffers (chunk = %lld); lower "
@@ -556,6 +563,7 @@ int mr_calc_toep_impl(const mr_config *cfg, const mr_complex *d_phi2, const floa
             printf("[mr_aha] calc_toep: components %lld-%lld of %lld issued\n", q0, q0 + qn - 1, Q);
     }
     MR_HIP_CHECK(hipStreamSynchronize(s));
+    b.done = true;
     return MR_SUCCESS;
 }
 
@@ -587,9 +595,10 @@ static int mr_calc_toep_from_psf_impl(const mr_config *cfg, const mr_complex *d_
     hipStream_t s = (hipStream_t)cfg->stream;
     const toep_geom tg = mr_toep_geom(cfg);
     const long long Qc = n_comp * tg.Nkz;
-    toep_bufs b;
+    toep_bufs b(s);
     if (cfg->is_masked) MR_TRY(mr_build_mask_rows(cfg, d_mask, s, &b.inv));
-    if (hipMalloc((void **)&b.nat, (size_t)tg.Ptr * Qc * sizeof(double2)) != hipSuccess) {
+    b.nat = (double2 *)mr_ws_get((size_t)tg.Ptr * Qc * sizeof(double2));
+    if (!b.nat) {
         (void)hipGetLastError();
         MR_FAIL(MR_ERR_ALLOC, "failed to allocate %lld scratch elements for mr_calc_toep_from_psf",
                 tg.Ptr * Qc);
@@ -606,6 +615,7 @@ static int mr_calc_toep_from_psf_impl(const mr_config *cfg, const mr_complex *d_
                        b.inv, (long long)cfg->num_masked, reinterpret_cast<float2 *>(d_out));
     MR_LAUNCH_CHECK("mr_k_toep_store");
     MR_HIP_CHECK(hipStreamSynchronize(s));
+    b.done = true;
     return MR_SUCCESS;
 }
 

@@ -124,3 +124,31 @@ def test_kernel_build_axes(mr, tt, n, M, chunk, monkeypatch):
     cfgm = mr.make_config(tt, n, L, phi2_dim=M, is_masked=True, num_masked=mask.numel())
     Km = mr.calc_toep(cfgm, dev(phi2), dev(traj), mask)
     assert torch.equal(torch.view_as_real(Km), torch.view_as_real(K.reshape(K.shape[0], -1)[:, mask]))
+
+
+def test_kept_scratch(mr):
+    """Builds of several sizes from several threads, each on its own stream,
+    equal the same builds one after another (a scratch block has one owner at a
+    time), and the memory kept between builds stays within the bound."""
+    from concurrent.futures import ThreadPoolExecutor
+    shapes = [("2D", (40, 36), 3), ("2D", (96, 80), 4), ("stack", (24, 20, 6), 3), ("3D", (16, 18, 14), 3)]
+    probs = [_problem(tt, n, L, 120, 40, 30 + i) for i, (tt, n, L) in enumerate(shapes)]
+    ins = [(dev(p[2]), dev(p[1])) for p in probs]
+    torch.cuda.synchronize()
+
+    def build(i, stream=None):
+        tt, n, L = shapes[i]
+        with torch.cuda.stream(stream):
+            return mr.calc_toep(mr.make_config(tt, n, L, stream=stream), *ins[i])
+
+    alone = [build(i) for i in range(4)]
+    free0 = torch.cuda.mem_get_info()[0]
+    streams = [torch.cuda.Stream() for _ in range(4)]
+    with ThreadPoolExecutor(4) as ex:
+        for _ in range(5):
+            got = list(ex.map(build, range(4), streams))
+            for a, b in zip(alone, got):
+                assert torch.equal(torch.view_as_real(a), torch.view_as_real(b))
+    torch.cuda.synchronize()
+    del got
+    assert free0 - torch.cuda.mem_get_info()[0] <= (4 << 30) + (64 << 20)
