@@ -23,6 +23,7 @@
 #include "mr_hip.hpp"
 #include "mr_aha/mr_aha_ext.h"
 #include "mr_xbd.hpp"
+#include "mr_xbd_rt.hpp"
 #include "mr_fft_ct.hpp"
 
 #include <cstdlib>
@@ -397,136 +398,8 @@ template <bool MASKED> static mr_bd_fn mr_bd_pick(int L, int TP)
 // Fused x pass (x-last pipeline)
 // ---------------------------------------------------------------------------
 
-// When the outer axes are transformed on the image side first, the x axis is
-// the last one: for one k-space row r = (ky, kz) (natural order) the forward
-// x-FFT, the block multiply of the row's Mx locations and the inverse x-FFT
-// need nothing outside the row. One workgroup takes the row for a group of up
-// to G coils of Y [Nx, R, V] (R = My*Mz rows, V = L * coils):
-//   load   the L*G pencils of Nx image columns, zero-padded to Mx in natural
-//          order (pad map of src/cuda/mr_kernels.cu:111-128)
-//   FFT    forward, radix stages in LDS
-//   block  v <- v B(k) at each of the Mx locations; the row's T*Mx kernel
-//          entries are read coalesced (centered kx runs contiguously except at
-//          the one wrap point) and shared, through L2, by the G coils and by
-//          the coil groups of the row, which are consecutive workgroups of
-//          one XCD (src/cuda/mr_kernels_bd.cu:74-139 for the walk)
-//   IFFT   inverse
-//   store  the Nx image columns back in place (crop of mr_kernels.cu:158-165)
-// Padded k-space never reaches HBM: per row and coil the pass moves 2*L*Nx
-// values plus the kernel row. Twiddles are read from the global table (L1
-// resident) so LDS holds exactly G*L*Mx values and two 80 KB workgroups can
-// share a CU.
-
-template <bool INV>
-__device__ __forceinline__ void mr_xbd_fft(float2 *A, const mr_fft_len<float> &f, int tp)
-{
-    int Ns = 1;
-    for (int s = 0; s < f.nst; ++s) {
-        const int RR = f.radix[s];
-        const mr_fdiv &md = f.mdiv[s], &nd = f.nsdiv[s];
-        switch (RR) {
-        case 2: mr_stage_reg<2, INV, float2, MR_XBD_THREADS, MR_XBD_EMAX>(A, f.tws, f.n, f.n, tp, Ns, md, nd); break;
-        case 3: mr_stage_reg<3, INV, float2, MR_XBD_THREADS, MR_XBD_EMAX>(A, f.tws, f.n, f.n, tp, Ns, md, nd); break;
-        case 4: mr_stage_reg<4, INV, float2, MR_XBD_THREADS, MR_XBD_EMAX>(A, f.tws, f.n, f.n, tp, Ns, md, nd); break;
-        case 5: mr_stage_reg<5, INV, float2, MR_XBD_THREADS, MR_XBD_EMAX>(A, f.tws, f.n, f.n, tp, Ns, md, nd); break;
-        case 6: mr_stage_reg<6, INV, float2, MR_XBD_THREADS, MR_XBD_EMAX>(A, f.tws, f.n, f.n, tp, Ns, md, nd); break;
-        case 7: mr_stage_reg<7, INV, float2, MR_XBD_THREADS, MR_XBD_EMAX>(A, f.tws, f.n, f.n, tp, Ns, md, nd); break;
-        case 10: mr_stage_reg<10, INV, float2, MR_XBD_THREADS, MR_XBD_EMAX>(A, f.tws, f.n, f.n, tp, Ns, md, nd); break;
-        default: mr_stage_reg<8, INV, float2, MR_XBD_THREADS, MR_XBD_EMAX>(A, f.tws, f.n, f.n, tp, Ns, md, nd); break;
-        }
-        Ns *= RR;
-    }
-}
-
-template <int L, bool MASKED>
-__global__ void __launch_bounds__(MR_XBD_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
-mr_k_xbd(float2 *__restrict__ Y, const float2 *__restrict__ ker, const int *__restrict__ inv,
-         long long kstride, mr_dims d, mr_fft_len<float> fx, mr_fdiv nxdiv, long long R, int G,
-         int ncoil, int ncg)
-{
-    constexpr int NW = MR_XBD_THREADS / 64;
-    extern __shared__ __align__(16) unsigned char mr_smem[];
-    float2 *A = reinterpret_cast<float2 *>(mr_smem);
-    const int Nx = d.n[0], Mx = d.m[0], cnx = d.c_n[0];
-    const long long q = mr_xcd_block(blockIdx.x, gridDim.x);
-    const long long r = q / ncg;
-    const int c0 = (int)(q - r * ncg) * G;
-    const int gn = (ncoil - c0 < G) ? ncoil - c0 : G;
-    const int tp = gn * L;
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // pencil pl = g*L + l of the workgroup is volume v = L*c0 + pl; every
-    // wavefront loads and stores whole pencils, so a pencil's base is uniform
-    const float2 *Yr = Y + (long long)Nx * r + (long long)Nx * R * L * c0;
-    const long long pstride = (long long)Nx * R;
-    const unsigned rowbytes = (unsigned)Nx * 8u;
-
-    for (int pl = wave; pl < tp; pl += NW) {
-        const __amdgpu_buffer_rsrc_t rs = mr_rsrc(Yr + pstride * pl, rowbytes);
-        float2 *Ap = A + pl * Mx;
-        for (int e = lane; e < Mx; e += 64) {
-            int s = e + cnx;
-            if (s >= Mx) s -= Mx;
-            Ap[e] = mr_bload(rs, (unsigned)s * 8u);   // s >= Nx reads zero: the padding
-        }
-    }
-    __syncthreads();
-    mr_xbd_fft<false>(A, fx, tp);
-
-    const int My = d.m[1];
-    const int jy = (int)(r % My), jz = (int)(r / My);
-    int ky = jy + d.c_m[1]; if (ky >= My) ky -= My;
-    int kz = jz + d.c_m[2]; if (kz >= d.m[2]) kz -= d.m[2];
-    const long long rowc = (long long)Mx * (ky + (long long)My * kz);
-    for (int w = threadIdx.x; w < gn * Mx; w += MR_XBD_THREADS) {
-        const int g = (int)mr_fdiv_q(fx.ndiv, (unsigned)w), e = w - g * Mx;
-        long long b;
-        if (MASKED) {
-            b = inv[e + (long long)Mx * r];
-        } else {
-            int kx = e + d.c_m[0];
-            if (kx >= Mx) kx -= Mx;
-            b = rowc + kx;
-        }
-        float2 *a = A + (size_t)g * L * Mx + e;
-        if (b < 0) {
-#pragma unroll
-            for (int l = 0; l < L; ++l) a[l * Mx] = make_float2(0.f, 0.f);
-        } else if (d.tri_upper) {
-            mr_bd_walk_g<L, true>(a, Mx, ker, kstride, (unsigned)(b * 8));
-        } else {
-            mr_bd_walk_g<L, false>(a, Mx, ker, kstride, (unsigned)(b * 8));
-        }
-    }
-    __syncthreads();
-    mr_xbd_fft<true>(A, fx, tp);
-
-    for (int pl = wave; pl < tp; pl += NW) {
-        const __amdgpu_buffer_rsrc_t rs = mr_rsrc(Yr + pstride * pl, rowbytes);
-        const float2 *Ap = A + pl * Mx;
-        for (int s = lane; s < Nx; s += 64) {
-            int e = s - cnx;
-            if (e < 0) e += Mx;
-            mr_bstore(rs, (unsigned)s * 8u, Ap[e]);
-        }
-    }
-}
-
-typedef void (*mr_xbd_fn)(float2 *, const float2 *, const int *, long long, mr_dims,
-                          mr_fft_len<float>, mr_fdiv, long long, int, int, int);
-
-template <bool MASKED> static mr_xbd_fn mr_xbd_pick(int L)
-{
-    switch (L) {
-#define MR_XBD_CASE(n) case n: return mr_k_xbd<n, MASKED>;
-        MR_XBD_CASE(1) MR_XBD_CASE(2) MR_XBD_CASE(3) MR_XBD_CASE(4)
-        MR_XBD_CASE(5) MR_XBD_CASE(6) MR_XBD_CASE(7) MR_XBD_CASE(8)
-        MR_XBD_CASE(9) MR_XBD_CASE(10) MR_XBD_CASE(11) MR_XBD_CASE(12)
-        MR_XBD_CASE(13) MR_XBD_CASE(14) MR_XBD_CASE(15) MR_XBD_CASE(16)
-#undef MR_XBD_CASE
-    default: return nullptr;
-    }
-}
+// mr_xbd_ct.hip holds the kernels compiled for common x lengths and ranks,
+// mr_xbd_rt.hip those for every other smooth length.
 
 // ---------------------------------------------------------------------------
 // Plan
@@ -558,8 +431,10 @@ struct mr_aha_plan_s {
     bool prof_on;
     int xbd_g;          // coils per workgroup of the fused x pass; 0 = separate passes
     size_t xbd_lds;     // its dynamic LDS bytes
-    mr_fdiv nxdiv;
-    mr_xbd_ct_fn xbd_ct;  // kernel specialised for (Mx, L), or null: mr_k_xbd
+    mr_xbd_ct_fn xbd_ct;  // kernel specialised for (Mx, L), or null: rt_fn
+    mr_rt_len rt;         // run-time-length kernel: plan, kernel, workgroup size
+    mr_xbd_rt_fn rt_fn;
+    int rt_nt;
     int xbd_nt;           // its workgroup size
     int tile[4];          // pencils per workgroup of Fo, Fy, Iy, Io (0: default rule)
     int no_wide;          // 1: no two-coil 1024-thread fused workgroups
@@ -665,6 +540,24 @@ static void mr_plan_free_buffers(mr_aha_plan p)
     p->d_inv = nullptr;
 }
 
+// Coils per workgroup of the run-time-length fused pass, `per` bytes of LDS a
+// coil: as many as keep two workgroups per CU (80 KB), rounded down to coil
+// pairs, which load each kernel entry once for both, and evened out over the
+// groups; else the pair in one workgroup of 1024 (160 KB), else one coil.
+// Where that leaves fewer than two workgroups per CU, smaller groups (a pair at
+// least): the rows are too few to fill the chip.
+static long long mr_xbd_rt_group(size_t per, int ncoil, long long rows)
+{
+    long long g = (long long)(81920 / per);
+    if (g < 2) return (2 * per <= 163840 && ncoil >= 2) ? 2 : 1;
+    g &= ~1LL;
+    if (g > ncoil) g = ncoil;
+    while (g > 2 && rows * mr_ceil_div(ncoil, g) < 512) g = (g + 1) / 2;
+    g = mr_ceil_div(ncoil, mr_ceil_div(ncoil, g));
+    if (g > 1 && (g & 1) && g < ncoil && (g + 1) * per <= 81920) ++g;
+    return g;
+}
+
 // Decide whether this plan runs the fused x pass: rank up to 16, an x length
 // made of the unrolled radices, and one coil's padded row within the LDS of a
 // workgroup. (Mx, L) pairs with a compile-time kernel use it. Default G: the
@@ -686,7 +579,7 @@ static int mr_xbd_setup(mr_aha_plan p)
         if (!mr_fft_unrolled(p->fx.radix[i])) return MR_SUCCESS;
     const long long per_elems = (long long)L * Mx;
     const size_t per = (size_t)per_elems * sizeof(float2);
-    if (per_elems > MR_XBD_EMAX) return MR_SUCCESS;
+    if (per_elems > MR_XBD_EMAX || !mr_rt_len_make(p->fx, &p->rt)) return MR_SUCCESS;
     // kernel entries are addressed with 32-bit byte offsets: one column, plus
     // up to L - 1 columns of scalar offset
     const long long kcol = cfg.is_masked ? (long long)cfg.num_masked : p->dims.pad_size;
@@ -707,13 +600,10 @@ static int mr_xbd_setup(mr_aha_plan p)
         if (gmax > ct_gmax) gmax = ct_gmax;
     } else if (p->kf != MR_KF_FP32) {
         return MR_SUCCESS;
-    } else {
-        mr_xbd_fn gf = cfg.is_masked ? mr_xbd_pick<true>(L) : mr_xbd_pick<false>(L);
-        if (!gf) return MR_SUCCESS;
-        fn = (const void *)gf;
     }
     if (gmax > cfg.n_coils) gmax = cfg.n_coils;
     long long g = (long long)(81920 / per);
+    if (!ct) g = mr_xbd_rt_group(per, cfg.n_coils, (long long)p->dims.m[1] * p->dims.m[2]);
     g = mr_env_ll("MR_AHA_HIP_XBD_G", g);
     if (g > gmax) g = gmax;
     if (g < 1) g = 1;
@@ -731,6 +621,12 @@ static int mr_xbd_setup(mr_aha_plan p)
         }
     }
     const size_t lds = per * (size_t)g;
+    if (!ct) {
+        p->rt_nt = lds <= 81920 ? 512 : 1024;
+        p->rt_fn = mr_xbd_rt_pick(L, cfg.is_masked != 0, p->rt_nt);
+        if (!p->rt_fn) return MR_SUCCESS;
+        fn = (const void *)p->rt_fn;
+    }
     if (lds > 65536 &&
         hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
             hipSuccess) {
@@ -776,7 +672,6 @@ static int mr_xbd_setup(mr_aha_plan p)
     p->xbd_mf = mf;
     p->xbd_pd = pd;
     p->xbd_nt = nt;
-    p->nxdiv = mr_fdiv_make((unsigned)p->dims.n[0]);
     return MR_SUCCESS;
 }
 
@@ -1217,7 +1112,7 @@ static int mr_execute_xlast(mr_aha_plan p, const float2 *x, const float2 *S, con
         if (blocks > 0x7fffffffLL)
             MR_FAIL(MR_ERR_UNSUPPORTED, "fused x pass: %lld workgroups exceed the launch limit",
                     blocks);
-        MR_GRID_CHECK(blocks, p->xbd_ct ? p->xbd_nt : MR_XBD_THREADS, "fused x pass");
+        MR_GRID_CHECK(blocks, p->xbd_ct ? p->xbd_nt : p->rt_nt, "fused x pass");
         if (p->xbd_ct) {
             // the matrix-core block step reads kernel entries two locations
             // per 16-byte load
@@ -1231,10 +1126,10 @@ static int mr_execute_xlast(mr_aha_plan p, const float2 *x, const float2 *S, con
                                p->ksc);
             MR_LAUNCH_CHECK("mr_k_xbd_ct");
         } else {
-            mr_xbd_fn fn = masked ? mr_xbd_pick<true>(L) : mr_xbd_pick<false>(L);
-            hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(MR_XBD_THREADS), p->xbd_lds, s, B,
-                               ker, p->d_inv, kstride, d, p->fx, p->nxdiv, R, G, nc, ncg);
-            MR_LAUNCH_CHECK("mr_k_xbd");
+            hipLaunchKernelGGL(p->rt_fn, dim3((unsigned)blocks), dim3((unsigned)p->rt_nt),
+                               p->xbd_lds, s, B, ker, p->d_inv, kstride, d, p->rt, p->fx.tws, R, G,
+                               nc, ncg);
+            MR_LAUNCH_CHECK("mr_k_xbd_rt");
         }
         MR_TRY(mr_prof_mark(p, MR_ST_BD));
     }

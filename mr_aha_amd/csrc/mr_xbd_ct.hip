@@ -1,6 +1,6 @@
 // Fused x pass specialised at compile time for the common x grid lengths.
 //
-// Same dataflow as mr_k_xbd (one k-space row, G coils, L ranks per
+// Same dataflow as mr_k_xbd_rt (one k-space row, G coils, L ranks per
 // workgroup: zero-padded load, forward x-FFT, block multiply, inverse x-FFT,
 // cropped store, in place), but the length N and the rank L are template
 // parameters. Every stage radix, stride and divisor is then a constant:
@@ -11,7 +11,7 @@
 // table (entry r*Ns + k - 1 of stage (R, Ns)).
 //
 // Instantiated for N in {256, 320, 384, 512, 640} and L in {4, 8, 16};
-// other shapes run mr_k_xbd.
+// other shapes run mr_k_xbd_rt.
 
 #include "mr_xbd.hpp"
 #include "mr_fft_ct.hpp"
