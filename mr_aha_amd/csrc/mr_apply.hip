@@ -1052,6 +1052,16 @@ static long long mr_zd_grid(long long ntiles)
     return ntiles < ncu ? ntiles : ncu;
 }
 
+// Outer passes on the run-time-length kernels (mr_axis_rt.hpp)? The forward pass
+// of the lengths compiled with whole-line tiles is as fast without them where
+// the plane is made of whole lines (320 along z of 160^3, L=8, 8 coils: 1.80
+// against 1.82 ms; 2D 192x192, L=8, 12 coils: 29 against 37 us).
+static bool mr_outer_rt(int n, bool inverse, long long plane)
+{
+    const bool w16 = n == 256 || n == 320 || n == 384 || n == 512;
+    return inverse || !w16 || plane % 16 != 0;
+}
+
 // x-last pipeline for one coil group (coils coil0 .. coil0 + nc - 1):
 //   Fo   outer axis (z; y in 2D): S_c x_l, zero-pad, FFT      -> A [Nx, Ny, Mz, V]
 //   Fy   y-FFT, zero-padding the Ny rows (3D and stack)      -> B [Nx, My, Mz, V]
@@ -1091,7 +1101,12 @@ static int mr_execute_xlast(mr_aha_plan p, const float2 *x, const float2 *S, con
                                fo.tws, x, S, A, plane, N, L, nc, coil0, cno, nt);
             MR_LAUNCH_CHECK("mr_k_fo_dma");
         } else {
-            MR_TRY((mr_fft_pass_ct<false>(fo, ld, st, plane * V, 0, txo, s, "Fo")));
+            int rc = MR_SUCCESS;
+            const mr_ax_z az{x, S, A, nullptr, plane, N, No, cno, L, nc, coil0, 0};
+            if (mr_outer_rt(Mo, false, plane) && mr_axis_rt_z(fo, false, az, s, &rc))
+                MR_TRY(rc);
+            else
+                MR_TRY((mr_fft_pass_ct<false>(fo, ld, st, plane * V, 0, txo, s, "Fo")));
         }
         MR_TRY(mr_prof_mark(p, two ? MR_ST_F2 : MR_ST_F3));
     }
@@ -1154,7 +1169,12 @@ static int mr_execute_xlast(mr_aha_plan p, const float2 *x, const float2 *S, con
                                nt);
             MR_LAUNCH_CHECK("mr_k_io_dma");
         } else {
-            MR_TRY((mr_fft_pass_ct<true>(fo, ld, st, plane * L, (size_t)No, txi, s, "Io")));
+            int rc = MR_SUCCESS;
+            const mr_ax_z az{nullptr, S, A, out, plane, N, No, cno, L, nc, coil0, coil0 > 0 ? 1 : 0};
+            if (mr_outer_rt(Mo, true, plane) && mr_axis_rt_z(fo, true, az, s, &rc))
+                MR_TRY(rc);
+            else
+                MR_TRY((mr_fft_pass_ct<true>(fo, ld, st, plane * L, (size_t)No, txi, s, "Io")));
         }
         MR_TRY(mr_prof_mark(p, two ? MR_ST_I2 : MR_ST_I3));
     }
@@ -1206,7 +1226,12 @@ static int mr_execute_impl(mr_aha_plan p, const float2 *x, const float2 *S, cons
             mr_zmap zm{V, lgTXZ};
             mr_ld_sx_z ld{x, S, zm, NxNy, N, Nz, Nz, d.c_n[2], L, coil0};
             mr_st_z st{A, zm, NxNy, Nz};
-            MR_TRY((mr_fft_pass_ct<false>(p->fz, ld, st, NxNy * V, 0, 1 << lgTXZ, s, "Z1")));
+            int rc = MR_SUCCESS;
+            const mr_ax_z az{x, S, A, nullptr, NxNy, N, Nz, d.c_n[2], L, nc, coil0, 0};
+            if (mr_outer_rt(Nz, false, NxNy) && mr_axis_rt_z(p->fz, false, az, s, &rc))
+                MR_TRY(rc);
+            else
+                MR_TRY((mr_fft_pass_ct<false>(p->fz, ld, st, NxNy * V, 0, 1 << lgTXZ, s, "Z1")));
             MR_TRY(mr_prof_mark(p, MR_ST_F3));
             // F1: zero-padded x-FFT -> B [Mx, Ny, Nz, V]
             mr_ld_pad<float2, true> l1{A, 1, Mx, Nx, d.c_n[0]};
@@ -1268,7 +1293,13 @@ static int mr_execute_impl(mr_aha_plan p, const float2 *x, const float2 *S, cons
             mr_zmap zm{L, lgTXZ};
             mr_ld_z_coil ld{src, zm, NxNy, Nz, L, nc};
             mr_st_z_conj_sum st{out, S, zm, NxNy, N, Nz, Nz, d.c_n[2], coil0, coil0 > 0 ? 1 : 0};
-            MR_TRY((mr_fft_pass_ct<true>(p->fz, ld, st, NxNy * L, (size_t)Nz, 1 << lgTXZ, s, "Z2")));
+            int rc = MR_SUCCESS;
+            const mr_ax_z az{nullptr, S, src, out, NxNy, N, Nz, d.c_n[2], L, nc, coil0,
+                             coil0 > 0 ? 1 : 0};
+            if (mr_outer_rt(Nz, true, NxNy) && mr_axis_rt_z(p->fz, true, az, s, &rc))
+                MR_TRY(rc);
+            else
+                MR_TRY((mr_fft_pass_ct<true>(p->fz, ld, st, NxNy * L, (size_t)Nz, 1 << lgTXZ, s, "Z2")));
             MR_TRY(mr_prof_mark(p, MR_ST_I3));
         } else {
             // I1: inverse x-FFT, crop, conj(S) and coil sum -> out

@@ -259,6 +259,25 @@ template <> struct mr_trig<7> {
                                     -0.97492791218182360702, -0.78183148246802980871};
 };
 
+template <> struct mr_trig<11> {
+    static constexpr double c[11] = {1.0, 0.8412535328311812, 0.41541501300188644,
+                                     -0.142314838273285, -0.654860733945285, -0.9594929736144974,
+                                     -0.9594929736144975, -0.6548607339452852,
+                                     -0.14231483827328523, 0.41541501300188605, 0.8412535328311812};
+    static constexpr double s[11] = {0.0, 0.5406408174555976, 0.9096319953545183, 0.9898214418809328,
+                                     0.7557495743542583, 0.28173255684142967, -0.2817325568414294, -0.7557495743542582,
+                                     -0.9898214418809327, -0.9096319953545186, -0.5406408174555974};
+};
+template <> struct mr_trig<13> {
+    static constexpr double c[13] = {1.0, 0.8854560256532099, 0.5680647467311559, 0.120536680255323,
+                                     -0.35460488704253545, -0.7485107481711012, -0.970941817426052, -0.9709418174260521,
+                                     -0.7485107481711013, -0.3546048870425359, 0.1205366802553232, 0.5680647467311548,
+                                     0.88545602565321};
+    static constexpr double s[13] = {0.0, 0.4647231720437685, 0.8229838658936564, 0.992708874098054, 0.9350162426854148,
+                                     0.6631226582407952, 0.23931566428755768, -0.23931566428755743, -0.663122658240795,
+                                     -0.9350162426854147, -0.992708874098054, -0.822983865893657, -0.4647231720437684};
+};
+
 template <int RR, bool INV, typename V> __device__ __forceinline__ void bfly_odd(V *v)
 {
     using R = decltype(V::x);
@@ -396,11 +415,15 @@ __device__ __forceinline__ void mr_stage_any(const V *__restrict__ A, V *__restr
         const int q = rem - j * RR;
         const int k = j % Ns;
         const V *a = A + p * ns + j;
-        const long long base = (long long)(k + Ns * q) * stride;
+        // exponent (k + Ns q) stride r mod n, stepped instead of divided
+        const int step = (int)((long long)(k + Ns * q) * stride % n);
+        int idx = 0;
         V acc = cmake<V>(0, 0);
         for (int r = 0; r < RR; ++r) {
-            V w = tw[(int)((base * r) % n)];
+            const V w = tw[idx];
             acc = cadd(acc, INV ? cmulc(w, a[r * m]) : cmul(w, a[r * m]));
+            idx += step;
+            if (idx >= n) idx -= n;
         }
         B[p * ns + (j / Ns) * Ns * RR + k + q * Ns] = acc;
     }

@@ -6,6 +6,7 @@
 // twiddle table (entry r*Ns + k - 1 of stage (R, Ns)).
 #pragma once
 
+#include "mr_axis_rt.hpp"
 #include "mr_hip.hpp"
 
 #include <type_traits>
@@ -889,8 +890,42 @@ int mr_fft_pass_ct_n(const mr_fft_len<float> &f, const Load &ld, const Store &st
     return MR_SUCCESS;
 }
 
+// y passes as the run-time-length kernels take them (mr_axis_rt.hpp): the
+// load's source column and the store's destination column.
+template <class Load> struct mr_ax_src { static constexpr bool kOk = false; };
+template <> struct mr_ax_src<mr_ld_pad<float2, false>> {
+    static constexpr bool kOk = true;
+    static void fill(mr_ax_y &a, const mr_ld_pad<float2, false> &l)
+    {
+        a.in = l.in; a.I = l.I; a.n_in = l.Ns; a.c_in = l.c;
+    }
+};
+template <> struct mr_ax_src<mr_ld_axis<float2, false>> {
+    static constexpr bool kOk = true;
+    static void fill(mr_ax_y &a, const mr_ld_axis<float2, false> &l)
+    {
+        a.in = l.in; a.I = l.I; a.n_in = l.n; a.c_in = 0;
+    }
+};
+template <class Store> struct mr_ax_dst { static constexpr bool kOk = false; };
+template <> struct mr_ax_dst<mr_st_axis<float2, false>> {
+    static constexpr bool kOk = true;
+    static void fill(mr_ax_y &a, const mr_st_axis<float2, false> &t)
+    {
+        a.out = t.out; a.n_out = t.n; a.c_out = 0;
+    }
+};
+template <> struct mr_ax_dst<mr_st_crop<float2, false>> {
+    static constexpr bool kOk = true;
+    static void fill(mr_ax_y &a, const mr_st_crop<float2, false> &t)
+    {
+        a.out = t.out; a.n_out = t.Ns; a.c_out = t.c;
+    }
+};
+
 // FP32 axis pass: the compile-time kernel for lengths 56, 256, 320, 384, 512
-// and 640 (MR_AHA_HIP_FFT_CT=0 turns it off), mr_fft_pass otherwise.
+// and 640 (MR_AHA_HIP_FFT_CT=0 turns it off); y passes of other lengths on the
+// run-time-length kernels (mr_axis_rt.hpp) where they can, mr_fft_pass otherwise.
 template <bool INV, class Load, class Store>
 int mr_fft_pass_ct(const mr_fft_len<float> &f, const Load &ld, const Store &st, long long npencil,
                    size_t acc_per_pencil, int want_tx, hipStream_t stream, const char *name)
@@ -904,6 +939,13 @@ int mr_fft_pass_ct(const mr_fft_len<float> &f, const Load &ld, const Store &st, 
 #undef MR_CT_LEN
         default: break;
         }
+    }
+    if constexpr (mr_ax_src<Load>::kOk && mr_ax_dst<Store>::kOk) {
+        mr_ax_y a;
+        mr_ax_src<Load>::fill(a, ld);
+        mr_ax_dst<Store>::fill(a, st);
+        int rc = MR_SUCCESS;
+        if (npencil > 0 && mr_axis_rt_y(f, INV, a, npencil, stream, &rc)) return rc;
     }
     return mr_fft_pass<float, INV>(f, ld, st, npencil, acc_per_pencil, want_tx, stream, name);
 }
