@@ -805,6 +805,8 @@ extern "C" MR_EXPORT int mr_aha_plan_destroy(mr_aha_plan plan)
 
 int mr_bdt_launch(const mr_dims &d, float2 *K, const float2 *ker, const int *inv,
                   long long kstride, int nc, bool masked, hipStream_t s);
+bool mr_bdm_launch(const mr_dims &d, float2 *K, const float2 *ker, const int *inv,
+                   long long kstride, int nc, bool masked, hipStream_t s, int *rc);
 
 static int mr_blockdiag(mr_aha_plan p, float2 *K, int nc, const float2 *ker)
 {
@@ -833,7 +835,10 @@ static int mr_blockdiag(mr_aha_plan p, float2 *K, int nc, const float2 *ker)
         MR_LAUNCH_CHECK("mr_k_bd");
         return MR_SUCCESS;
     }
-    // ranks without a compiled kernel: the tiled kernel (LDS panels)
+    // ranks without a compiled kernel: matrix cores or the tiled
+    // kernel, by rank and coils
+    int rc;
+    if (mr_bdm_launch(d, K, ker, p->d_inv, kstride, nc, masked, p->stream, &rc)) return rc;
     return mr_bdt_launch(d, K, ker, p->d_inv, kstride, nc, masked, p->stream);
 }
 

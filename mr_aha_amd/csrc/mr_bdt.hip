@@ -1,5 +1,7 @@
-// Block multiply for ranks above the compiled ones (L = 17 .. 512), in place
-// over the padded k-space grids of the separate-pass route.
+// Block multiply for ranks above the compiled ones (L = 17 .. 512) where the
+// matrix-core kernel (mr_bdm.hip) does not apply: ranks above 80, and lower ones
+// with few coils. In place over the padded k-space grids of the separate-pass
+// route.
 //
 // Same operation as the reference's tiled kernels
 // (src/cuda/mr_kernels_bdt.cu:218-416): at every grid location
@@ -132,12 +134,10 @@ __device__ __forceinline__ void bdt_run_rows(float2 (&y)[NCB][OPT], const float2
     if (r < r1) bdt_step<OPT, NCB, true>(y, a0, vr + (size_t)r * NCB * BDT_TP);
 }
 
-// Work-items per workgroup at most: 1024, or 512 for the 12-coil batch, whose
-// accumulators need more than the 128 VGPRs a 1024-wide workgroup allows.
-constexpr int bdt_max_threads(int ncb) { return ncb >= 12 ? 512 : 1024; }
+constexpr int BDT_MAX_THREADS = 1024;
 
 template <int OPT, int NCB, bool MASKED>
-__global__ void __launch_bounds__(bdt_max_threads(NCB))
+__global__ void __launch_bounds__(BDT_MAX_THREADS)
 mr_k_bdt(float2 *__restrict__ K, const float2 *__restrict__ ker, const int *__restrict__ inv,
          long long kstride, mr_dims d, int ncoil, int ng, int nbat)
 {
@@ -246,8 +246,6 @@ template <bool MASKED> mr_bdt_fn bdt_fn(int opt, int ncb)
     case 402: return mr_k_bdt<4, 2, MASKED>;
     case 404: return mr_k_bdt<4, 4, MASKED>;
     case 206: return mr_k_bdt<2, 6, MASKED>;
-    case 208: return mr_k_bdt<2, 8, MASKED>;
-    case 212: return mr_k_bdt<2, 12, MASKED>;
     case 801: return mr_k_bdt<8, 1, MASKED>;
     default: return nullptr;
     }
@@ -264,7 +262,7 @@ int mr_bdt_launch(const mr_dims &d, float2 *K, const float2 *ker, const int *inv
     const int L = d.L;
     MR_REQUIRE(L >= 1 && L <= 512, "block multiply: rank L = %d outside 1..512", L);
     MR_REQUIRE(nc >= 1, "block multiply: %d coils", nc);
-    const long long cap = mr_env_ll("MR_AHA_HIP_BDT_NCB", 12);
+    const long long cap = mr_env_ll("MR_AHA_HIP_BDT_NCB", 6);
     const long long want_opt = mr_env_ll("MR_AHA_HIP_BDT_OPT", 0);
     int opt, ncb;
     if (L > 256) {
@@ -277,7 +275,7 @@ int mr_bdt_launch(const mr_dims &d, float2 *K, const float2 *ker, const int *inv
                                                      160 * 1024);
         const int fit = std::max(1, (int)(budget / ((long long)L * BDT_TP * sizeof(float2))));
         const int lim = (int)std::min<long long>(std::min<long long>(cap, nc), fit);
-        const int batches[] = {12, 8, 6, 4, 2, 1};
+        const int batches[] = {6, 4, 2, 1};
         ncb = 1;
         for (int b : batches)
             if (b <= lim) { ncb = b; break; }
@@ -289,7 +287,7 @@ int mr_bdt_launch(const mr_dims &d, float2 *K, const float2 *ker, const int *inv
         if (want_opt == 2 || want_opt == 4) opt = (int)want_opt;
         // a compiled form whose workgroup holds all output groups
         while (!bdt_fn<false>(opt, ncb) ||
-               BDT_TP * (((L + opt - 1) / opt + 3) / 4 * 4) > bdt_max_threads(ncb)) {
+               BDT_TP * (((L + opt - 1) / opt + 3) / 4 * 4) > BDT_MAX_THREADS) {
             if (opt == 2 && bdt_fn<false>(4, ncb)) opt = 4;
             else if (ncb > 1) { ncb = ncb > 4 ? 4 : ncb / 2; opt = 4; }
             else break;
@@ -300,7 +298,7 @@ int mr_bdt_launch(const mr_dims &d, float2 *K, const float2 *ker, const int *inv
                ncb);
     const int ng = (L + opt - 1) / opt;
     const int threads = BDT_TP * ((ng + 3) / 4 * 4);   // whole wavefronts
-    MR_REQUIRE(threads <= bdt_max_threads(ncb), "block multiply: %d work-items", threads);
+    MR_REQUIRE(threads <= BDT_MAX_THREADS, "block multiply: %d work-items", threads);
     const size_t lds = (size_t)ncb * L * BDT_TP * sizeof(float2);
     if (lds > 65536 &&
         hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
