@@ -4,6 +4,7 @@
 
 #include <hipcub/hipcub.hpp>
 
+#include <algorithm>
 #include <cmath>
 
 void mr_grid_setup(mr_grid *g, int d, const int *M, double eps)
@@ -351,8 +352,10 @@ int mr_grid_samples_build(const mr_grid &g, const float *traj, long long Ntrajs,
 // strengths (PER_SAMPLE false) the weights of consecutive samples of one
 // readout are summed first and the CB strengths applied once per run; the
 // strengths of a key are contiguous and uniform over the wavefront, so they
-// come through the scalar cache. The first segment of a tile is stored to the
-// fine grid, later ones to `part`, which mr_k_spread_sum adds in order.
+// come through the scalar cache. Per-sample strengths would each wait for it, so
+// they are staged in LDS with the kernel values (16 sets 215 -> 92 us). The
+// first segment of a tile is stored to the fine grid, later ones to `part`,
+// which mr_k_spread_sum adds in order.
 //
 // The bound is the FP64 arithmetic of the weights and strengths once the work
 // is even. A tile at the centre of radial samples has a thousand times the
@@ -361,17 +364,19 @@ int mr_grid_samples_build(const mr_grid &g, const float *traj, long long Ntrajs,
 // (512 x 512 samples, 36 sets) 2.58 -> 0.34 ms, 192x192x32 L=8 (1152 sets)
 // 26.9 -> 3.8 ms, of which the 10.9 GB of output take 2.0, 96^3 L=4 (4000 x
 // 192 samples) 49.7 -> 3.8 ms (9.1 GB, 1.7 ms); per sample, 128 x 384 samples
-// onto 768x768, 4 sets, 1.26 -> 0.09 ms.
+// onto 384x384, 4 sets, 1.26 -> 0.09 ms.
 // ---------------------------------------------------------------------------
 
 // LDS of one wavefront: 64 samples' kernel values (the odd stride keeps the
 // staging writes off each other's banks), their keys, and the tile's ranges.
-template <int D> struct mr_spread_lds {
+// SC: strengths staged beside them.
+template <int D, int SC = 0> struct mr_spread_lds {
     static constexpr int BS = (D == 2) ? 8 : 4;
     static constexpr int STR = D * BS + 1;
     double w[64 * STR];
     int key[64];
     int base[64], end[64];
+    double2 c[SC > 0 ? 64 * SC : 1];   // [slot][set]
 };
 
 template <int D, int CB, bool PER_SAMPLE>
@@ -381,7 +386,7 @@ mr_k_spread(mr_grid g, const int *__restrict__ i0s, const int *__restrict__ rds,
             const int2 *__restrict__ ext, long long next, const double2 *__restrict__ str, int qs,
             int q0, int Q, double2 *__restrict__ fine, double2 *__restrict__ part)
 {
-    using lds_t = mr_spread_lds<D>;
+    using lds_t = mr_spread_lds<D, PER_SAMPLE ? CB : 0>;
     constexpr int BS = lds_t::BS, STR = lds_t::STR;
     __shared__ lds_t sh4[4];
     const int lane = threadIdx.x & 63;
@@ -463,6 +468,19 @@ mr_k_spread(mr_grid g, const int *__restrict__ i0s, const int *__restrict__ rds,
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        if constexpr (PER_SAMPLE) {
+            // the strengths of the staged samples, all loads in flight at once
+            double2 v[CB];
+#pragma unroll
+            for (int n = 0; n < CB; ++n) {
+                const int f = lane + 64 * n, j = f / CB, q = f % CB;
+                v[n] = j < cnt ? strq[(long long)sh.key[j] * qs + q] : make_double2(0.0, 0.0);
+            }
+#pragma unroll
+            for (int n = 0; n < CB; ++n) sh.c[lane + 64 * n] = v[n];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
         const int key = sh.key[lane];
         auto weight = [&](int j) {
             const double *ws = sh.w + j * STR;
@@ -470,8 +488,8 @@ mr_k_spread(mr_grid g, const int *__restrict__ i0s, const int *__restrict__ rds,
             if (D == 3) v *= ws[2 * BS + p[2]];
             return v;
         };
-        auto apply = [&](double wv, int ky) {
-            const double2 *c = strq + (long long)ky * qs;
+        auto apply = [&](double wv, int ky) {   // ky: the slot, or the readout of a run
+            const double2 *c = PER_SAMPLE ? sh.c + ky * CB : strq + (long long)ky * qs;
 #pragma unroll
             for (int q = 0; q < CB; ++q) {
                 const double2 v = c[q];
@@ -496,7 +514,7 @@ mr_k_spread(mr_grid g, const int *__restrict__ i0s, const int *__restrict__ rds,
                 if (j0 + j >= cnt) break;
                 wsum += wv[j];
                 if ((ends >> (j0 + j)) & 1) {
-                    apply(wsum, __builtin_amdgcn_readlane(key, j0 + j));
+                    apply(wsum, PER_SAMPLE ? j0 + j : __builtin_amdgcn_readlane(key, j0 + j));
                     wsum = 0.0;
                 }
             }
@@ -554,7 +572,9 @@ static int mr_spread_launch(const mr_grid &g, const mr_grid_samples &s, const do
                             int q0, int Q, double2 *fine, double2 *part, hipStream_t stream)
 {
     // strengths per wavefront: the fewest that keep the number of chunks of 16
-    const int chunks = (Q + 15) / 16, per = (Q + chunks - 1) / chunks;
+    // (of 8 where they are staged in LDS)
+    constexpr int CMAX = PER_SAMPLE ? 8 : 16;
+    const int chunks = (Q + CMAX - 1) / CMAX, per = (Q + chunks - 1) / chunks;
     const long long blocks = mr_ceil_div(g.nbins + s.next, 4);
 #define MR_SPREAD(CB)                                                                             \
     do {                                                                                          \
@@ -566,8 +586,10 @@ static int mr_spread_launch(const mr_grid &g, const mr_grid_samples &s, const do
     } while (0)
     if (per <= 4) MR_SPREAD(4);
     else if (per <= 8) MR_SPREAD(8);
-    else if (per <= 12) MR_SPREAD(12);
-    else MR_SPREAD(16);
+    else if constexpr (!PER_SAMPLE) {
+        if (per <= 12) MR_SPREAD(12);
+        else MR_SPREAD(16);
+    }
 #undef MR_SPREAD
     MR_LAUNCH_CHECK("mr_k_spread");
     if (s.next > 0) {
@@ -592,58 +614,82 @@ int mr_grid_spread_samples(const mr_grid &g, const mr_grid_samples &s, const dou
                     : mr_spread_launch<3, true>(g, s, str, Q, 0, Q, fine, part, stream);
 }
 
-// Type-2 interpolation, one thread per (sorted sample, set q).
-template <int D>
-__global__ void mr_k_interp(mr_grid g, const int *__restrict__ i0s, const double *__restrict__ wts,
-                            long long n, const double2 *__restrict__ fine, int Q,
-                            double2 *__restrict__ out)
+// Type-2 interpolation. Eight lanes share a sample and QT sets: lane k reads
+// column k (and k + 8) of every row the sample touches, so a load of the
+// wavefront takes eight runs of w values instead of 64 values of 64 lines,
+// whose addresses bounded it; the sets share weights and addressing, and their
+// loads overlap. The lanes' sums are added at the end. 128 x 384 samples onto
+// 16 grids of 384 x 384, w = 7: 124 -> 37 us.
+template <int D, int QT>
+__global__ void __launch_bounds__(256)
+mr_k_interp(mr_grid g, const int *__restrict__ i0s, const double *__restrict__ wts, long long n,
+            const double2 *__restrict__ fine, int Q, double2 *__restrict__ out, long long base)
 {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int q = blockIdx.y;
-    if (i >= n || q >= Q) return;
+    const long long id = base * 256 + (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long i = id >> 3;
+    const int k = (int)id & 7, q0 = blockIdx.y * QT;
+    if (i >= n) return;   // all eight lanes of a sample
     const int w = g.w;
-    const double2 *f = fine + (long long)q * g.nfine;
+    const double2 *f[QT];
+#pragma unroll
+    for (int q = 0; q < QT; ++q) f[q] = fine + (long long)(q0 + q < Q ? q0 + q : Q - 1) * g.nfine;
     const double *wx = wts + (i * D + 0) * w;
     const double *wy = wts + (i * D + 1) * w;
     const double *wz = (D == 3) ? wts + (i * D + 2) * w : nullptr;
     const int ix = i0s[i * 3], iy = i0s[i * 3 + 1], iz = i0s[i * 3 + 2];
-    double ar = 0.0, ai = 0.0;
+    double2 a[QT];
+#pragma unroll
+    for (int q = 0; q < QT; ++q) a[q] = make_double2(0.0, 0.0);
     const int nz = (D == 3) ? w : 1;
-    for (int kz = 0; kz < nz; ++kz) {
-        int gz = 0;
-        double fz = 1.0;
-        if (D == 3) {
-            gz = iz + kz;
-            if (gz >= g.nf[2]) gz -= g.nf[2];
-            fz = wz[kz];
-        }
-        for (int ky = 0; ky < w; ++ky) {
-            int gy = iy + ky;
-            if (gy >= g.nf[1]) gy -= g.nf[1];
-            const double fy = fz * wy[ky];
-            const double2 *row = f + (long long)g.nf[0] * (gy + (long long)g.nf[1] * gz);
-            for (int kx = 0; kx < w; ++kx) {
-                int gx = ix + kx;
-                if (gx >= g.nf[0]) gx -= g.nf[0];
-                const double wv = fy * wx[kx];
-                const double2 v = row[gx];
-                ar += wv * v.x;
-                ai += wv * v.y;
+    for (int kx = k; kx < w; kx += 8) {
+        int gx = ix + kx;
+        if (gx >= g.nf[0]) gx -= g.nf[0];
+        const double fx = wx[kx];
+        for (int kz = 0; kz < nz; ++kz) {
+            int gz = 0;
+            double fz = fx;
+            if (D == 3) {
+                gz = iz + kz;
+                if (gz >= g.nf[2]) gz -= g.nf[2];
+                fz = fx * wz[kz];
+            }
+#pragma unroll 2
+            for (int ky = 0; ky < w; ++ky) {
+                int gy = iy + ky;
+                if (gy >= g.nf[1]) gy -= g.nf[1];
+                const double wv = fz * wy[ky];
+                const long long o = gx + (long long)g.nf[0] * (gy + (long long)g.nf[1] * gz);
+#pragma unroll
+                for (int q = 0; q < QT; ++q) {
+                    const double2 v = f[q][o];
+                    a[q].x += wv * v.x;
+                    a[q].y += wv * v.y;
+                }
             }
         }
     }
-    out[i * Q + q] = make_double2(ar, ai);
+#pragma unroll
+    for (int q = 0; q < QT; ++q) {
+#pragma unroll
+        for (int o = 1; o < 8; o <<= 1) {
+            a[q].x += __shfl_xor(a[q].x, o);
+            a[q].y += __shfl_xor(a[q].y, o);
+        }
+        if (k == q && q0 + q < Q) out[i * Q + q0 + q] = a[q];
+    }
 }
 
 int mr_grid_interp(const mr_grid &g, const mr_grid_samples &s, const double2 *fine, int Q,
                    double2 *out, hipStream_t stream)
 {
-    const dim3 grid((unsigned)mr_ceil_div(s.n, 256), (unsigned)Q);
-    if (g.d == 2)
-        hipLaunchKernelGGL(mr_k_interp<2>, grid, dim3(256), 0, stream, g, s.i0, s.wt, s.n, fine, Q, out);
-    else
-        hipLaunchKernelGGL(mr_k_interp<3>, grid, dim3(256), 0, stream, g, s.i0, s.wt, s.n, fine, Q, out);
-    MR_LAUNCH_CHECK("mr_k_interp");
+    constexpr int QT = 4;
+    const long long blocks = mr_ceil_div(s.n, 32), step = mr_max_blocks(256);
+    auto *fn = g.d == 2 ? mr_k_interp<2, QT> : mr_k_interp<3, QT>;
+    for (long long b0 = 0; b0 < blocks; b0 += step) {   // a dispatch counts 2^32 work-items
+        hipLaunchKernelGGL(fn, dim3((unsigned)std::min(step, blocks - b0), (unsigned)((Q + QT - 1) / QT)),
+                           dim3(256), 0, stream, g, s.i0, s.wt, s.n, fine, Q, out, b0);
+        MR_LAUNCH_CHECK("mr_k_interp");
+    }
     return MR_SUCCESS;
 }
 

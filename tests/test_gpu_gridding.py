@@ -152,3 +152,28 @@ def test_kept_scratch(mr):
     torch.cuda.synchronize()
     del got
     assert free0 - torch.cuda.mem_get_info()[0] <= (4 << 30) + (64 << 20)
+
+
+@pytest.mark.parametrize("tt,n,L,C", [("2D", (33, 27), 3, 5), ("2D", (17, 40), 1, 7),
+                                      ("stack", (19, 24, 5), 2, 3), ("3D", (14, 11, 9), 2, 3)])
+def test_nufft_coil_batches(mr, monkeypatch, tt, n, L, C):
+    """Coils through the comparator one at a time, a few at a time (a last batch
+    that is smaller) and all at once: the same sums in the same order, against
+    the exact NUDFT at the gridding's accuracy (1e-5) and each other (1e-6)."""
+    from oracle import nudft
+    print(f"[gridding] nufft coil batches {tt} {n} L={L} C={C}", flush=True)
+    g, traj, phi2 = _problem(tt, n, L, 23, 2 * max(n[:2]), L + C)
+    rng = np.random.default_rng(L)
+    cplx = lambda s: (rng.standard_normal(s) + 1j * rng.standard_normal(s)).astype(np.complex64)  # noqa: E731
+    x, S = cplx((L,) + g.img_shape()), cplx((C,) + g.img_shape())
+    ref = nudft.aha_nudft(g, x, S, phi2, traj)
+    cfg = mr.make_config(tt, n, L, n_coils=C)
+    outs = []
+    for mb in ("0", "1", "1024"):
+        monkeypatch.setenv("MR_AHA_HIP_NU_MB", mb)
+        with mr.create_op(cfg, dev(S), dev(phi2), dev(traj), method="nufft") as op:
+            for _ in range(2):   # the second pass finds the first one's buffers
+                outs.append(op(dev(x)).cpu().numpy())
+    assert rel(outs[0], ref) < 1e-5
+    for y in outs[1:]:
+        assert rel(y, outs[0]) < 1e-6
