@@ -15,7 +15,7 @@
 struct mr_d24 {
     unsigned mul, shr;
 };
-inline mr_d24 mr_d24_make(unsigned d)
+__host__ __device__ inline constexpr mr_d24 mr_d24_make(unsigned d)
 {
     unsigned l = 0;
     while ((1u << l) < d) ++l;
