@@ -850,10 +850,21 @@ static int mr_blockdiag(mr_aha_plan p, float2 *K, int nc, const float2 *ker)
 // global_load_lds_dwordx4 while the previous tile is transformed and
 // stored. The first radix stage reads the loaded rows and writes the work
 // buffer, so the next tile's rows can land as soon as it is done.
+// z lengths 16 .. 64 in steps of 8, whole apply against the run-time-length
+// passes: 192x192, L=16, 16 coils: 16 partitions 7.64 -> 6.80 ms, 32 14.1 ->
+// 13.7, 64 27.4 -> 26.8; 160x160, L=16, 4 coils: 16 1.20 -> 1.04 ms, 64 4.20 ->
+// 4.15.
 // ---------------------------------------------------------------------------
 
 constexpr int MR_ZD_LB = 8;              // ranks per tile
+// up to this length two workgroups per CU, by LDS and 64 registers (224x224x16,
+// L=8, 10 coils 2.74 -> 2.61 ms, x24 3.99 -> 3.90; 32 spills and gains nothing)
+constexpr int MR_ZD_TWO = 24;
 constexpr int MR_ZD_PT = 16 * MR_ZD_LB;  // pencils per tile
+// All twiddles of a butterfly, from the table: in scalar registers they cost no
+// more than the first with its powers, and the apply's error against FP64 falls
+// (320x320x56, L=16, 12 coils 4.1e-7 -> 3.5e-7; at equal speed, 39.3 -> 39.2 ms).
+constexpr int MR_ZD_WN = 7;
 // LDS stride of one rank's N rows of 16 xy, padded by one row so that the
 // four ranks a wavefront reads at once start on alternate bank halves
 template <int N> constexpr int mr_zd_xs() { return N * 16 + 16; }
@@ -865,7 +876,7 @@ template <int N> constexpr int mr_zd_xs() { return N * 16 + 16; }
 // LDS buffers), and the next tile's x rows while the last coil is. Output
 // [plane, N, V] (v = l + L c) as mr_st_z.
 template <int N>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(1024, N <= MR_ZD_TWO ? 8 : 4)
 mr_k_fo_dma(const float2 *tws, const float2 *__restrict__ x, const float2 *__restrict__ S,
             float2 *__restrict__ out, long long NxNy, long long Nimg, int L, int nc, int coil0,
             int cnz, long long ntiles)
@@ -876,8 +887,8 @@ mr_k_fo_dma(const float2 *tws, const float2 *__restrict__ x, const float2 *__res
     __shared__ __align__(16) float2 Bs0[N * 16];         // [z][xy], even coils
     __shared__ __align__(16) float2 Bs1[N * 16];         // odd coils
     __shared__ __align__(16) float2 A[N * PT];           // [e][rank * 16 + xy]
-    float2 w[MR_EP_NST][MR_EP_KMAX];
-    mr_ep_twload<N, 0, NT, PT>(w, mr_tw_buf{mr_rsrc(tws, (unsigned)N * 8u)});
+    mr_ep_tw<MR_ZD_WN> w[MR_EP_NST];
+    mr_ep_twload<N, 0, NT, PT, MR_ZD_WN>(w, mr_tw_buf{mr_rsrc(tws, (unsigned)N * 8u)});
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nlb = L / MR_ZD_LB;
@@ -903,7 +914,7 @@ mr_k_fo_dma(const float2 *tws, const float2 *__restrict__ x, const float2 *__res
     auto coil = [&](long long t, int c, const float2 *bcur, float2 *bnext) {
         __builtin_amdgcn_s_waitcnt(0);   // this wavefront's row loads
         __syncthreads();                 // everyone's
-        mr_ep_stage<N, 0, false, NT, PT, true>(A, w[0], [&](int pp, int e) {
+        mr_ep_stage<N, 0, false, NT, PT, true, MR_ZD_WN>(A, w[0], [&](int pp, int e) {
             int z = e + cnz;
             if (z >= N) z -= N;
             const int xy = pp & 15;
@@ -911,7 +922,7 @@ mr_k_fo_dma(const float2 *tws, const float2 *__restrict__ x, const float2 *__res
         });
         if (c + 1 < nc) fill(t, c + 1, bnext, false);
         else if (t + gridDim.x < ntiles) fill(t + gridDim.x, 0, bnext, true);
-        mr_ep_fft<N, 1, false, NT, PT>(A, w);
+        mr_ep_fft<N, 1, false, NT, PT, MR_ZD_WN>(A, w);
         const long long v = (t % nlb) * MR_ZD_LB + (p >> 4) + (long long)L * c;
         float2 *o = out + (t / nlb) * 16 + (p & 15) + NxNy * (long long)N * v;
         for (int e = threadIdx.x / PT; e < N; e += NT / PT) o[NxNy * e] = A[e * PT + p];
@@ -938,7 +949,7 @@ mr_k_fo_dma(const float2 *tws, const float2 *__restrict__ x, const float2 *__res
 // `accumulate`) after the last coil. The S rows of consecutive coils
 // alternate between two LDS buffers.
 template <int N>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(1024, N <= MR_ZD_TWO ? 8 : 4)
 mr_k_io_dma(const float2 *tws, const float2 *__restrict__ in, const float2 *__restrict__ S,
             float2 *__restrict__ out, long long NxNy, long long Nimg, int L, int nc, int coil0,
             int cnz, int accumulate, long long ntiles)
@@ -950,8 +961,8 @@ mr_k_io_dma(const float2 *tws, const float2 *__restrict__ in, const float2 *__re
     __shared__ __align__(16) float2 Bs0[N * 16];         // [z][xy], even coils
     __shared__ __align__(16) float2 Bs1[N * 16];         // odd coils
     __shared__ __align__(16) float2 W[N * PT];           // [e][rank * 16 + xy]
-    float2 w[MR_EP_NST][MR_EP_KMAX];
-    mr_ep_twload<N, 0, NT, PT>(w, mr_tw_buf{mr_rsrc(tws, (unsigned)N * 8u)});
+    mr_ep_tw<MR_ZD_WN> w[MR_EP_NST];
+    mr_ep_twload<N, 0, NT, PT, MR_ZD_WN>(w, mr_tw_buf{mr_rsrc(tws, (unsigned)N * 8u)});
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nlb = L / MR_ZD_LB;
@@ -981,7 +992,7 @@ mr_k_io_dma(const float2 *tws, const float2 *__restrict__ in, const float2 *__re
     auto coil = [&](long long t, int c, const float2 *bcur, float2 *bnext) {
         __builtin_amdgcn_s_waitcnt(0);   // this wavefront's row loads
         __syncthreads();                 // everyone's
-        mr_ep_stage<N, 0, true, NT, PT, true>(W, w[0], [&](int pp, int e) {
+        mr_ep_stage<N, 0, true, NT, PT, true, MR_ZD_WN>(W, w[0], [&](int pp, int e) {
             return Bx[(pp >> 4) * XS + e * 16 + (pp & 15)];
         });
         long long tn = t;
@@ -991,7 +1002,7 @@ mr_k_io_dma(const float2 *tws, const float2 *__restrict__ in, const float2 *__re
             tn = t + gridDim.x;
         }
         if (tn < ntiles) fill(tn, cn, bnext);
-        mr_ep_fft<N, 1, true, NT, PT>(W, w);
+        mr_ep_fft<N, 1, true, NT, PT, MR_ZD_WN>(W, w);
 #pragma unroll
         for (int k = 0; k < KE; ++k) {
             int z = e0 + 8 * k + cnz;
@@ -1032,19 +1043,38 @@ mr_k_io_dma(const float2 *tws, const float2 *__restrict__ in, const float2 *__re
     }
 }
 
+typedef void (*mr_zd_fo_fn)(const float2 *, const float2 *, const float2 *, float2 *, long long,
+                            long long, int, int, int, int, long long);
+typedef void (*mr_zd_io_fn)(const float2 *, const float2 *, const float2 *, float2 *, long long,
+                            long long, int, int, int, int, int, long long);
+#define MR_ZD_EACH(K)                                                                            \
+    switch (n) {                                                                                 \
+    case 16: return K<16>;                                                                       \
+    case 24: return K<24>;                                                                       \
+    case 32: return K<32>;                                                                       \
+    case 40: return K<40>;                                                                       \
+    case 48: return K<48>;                                                                       \
+    case 56: return K<56>;                                                                       \
+    case 64: return K<64>;                                                                       \
+    default: return nullptr;                                                                     \
+    }
+static mr_zd_fo_fn mr_zd_fo(int n) { MR_ZD_EACH(mr_k_fo_dma) }
+static mr_zd_io_fn mr_zd_io(int n) { MR_ZD_EACH(mr_k_io_dma) }
+#undef MR_ZD_EACH
+
 // Run Fo / Io on the double-buffered kernels when the shape allows (z length
-// 56 = Mz = Nz, whole 16-position xy tiles, ranks in blocks of 8, 16-byte
+// Mz = Nz one of the compiled ones, whole 16-position xy tiles, ranks in blocks of 8, 16-byte
 // aligned arrays); false: use the one-tile passes.
 static bool mr_zd_ok(const mr_dims &d, int L, long long plane, const void *a, const void *b,
                      const void *c)
 {
-    return d.m[2] == 56 && d.n[2] == 56 && plane % 16 == 0 && L % MR_ZD_LB == 0 &&
+    return mr_zd_fo(d.m[2]) && d.n[2] == d.m[2] && plane % 16 == 0 && L % MR_ZD_LB == 0 &&
            d.image_size % 2 == 0 && (((unsigned long long)a | (unsigned long long)b |
                                       (unsigned long long)c) & 15) == 0 &&
            mr_env_ll("MR_AHA_HIP_ZDMA", 1) != 0;
 }
 
-static long long mr_zd_grid(long long ntiles)
+static long long mr_zd_grid(long long ntiles, int n = MR_ZD_TWO + 1)
 {
     static int ncu = 0;
     if (ncu == 0) {
@@ -1054,7 +1084,8 @@ static long long mr_zd_grid(long long ntiles)
                 hipSuccess || ncu <= 0)
             ncu = 256;
     }
-    return ntiles < ncu ? ntiles : ncu;
+    const long long most = (long long)ncu * (n <= MR_ZD_TWO ? 2 : 1);
+    return ntiles < most ? ntiles : most;
 }
 
 // Outer passes on the run-time-length kernels (mr_axis_rt.hpp)? The forward pass
@@ -1102,7 +1133,7 @@ static int mr_execute_xlast(mr_aha_plan p, const float2 *x, const float2 *S, con
         const int txo = (int)mr_env_ll("MR_AHA_HIP_FO_TX", p->tile[0] > 0 ? p->tile[0] : 1 << lgT);
         if (!two && mr_zd_ok(d, L, plane, x, S, A)) {
             const long long nt = (plane / 16) * (L / MR_ZD_LB);
-            hipLaunchKernelGGL(mr_k_fo_dma<56>, dim3((unsigned)mr_zd_grid(nt)), dim3(1024), 0, s,
+            hipLaunchKernelGGL(mr_zd_fo(Mo), dim3((unsigned)mr_zd_grid(nt, Mo)), dim3(1024), 0, s,
                                fo.tws, x, S, A, plane, N, L, nc, coil0, cno, nt);
             MR_LAUNCH_CHECK("mr_k_fo_dma");
         } else {
@@ -1169,7 +1200,7 @@ static int mr_execute_xlast(mr_aha_plan p, const float2 *x, const float2 *S, con
                                        p->tile[3] > 0 ? p->tile[3] : 1 << (lgT < 5 ? lgT : 5));
         if (!two && mr_zd_ok(d, L, plane, A, S, out)) {
             const long long nt = (plane / 16) * (L / MR_ZD_LB);
-            hipLaunchKernelGGL(mr_k_io_dma<56>, dim3((unsigned)mr_zd_grid(nt)), dim3(1024), 0, s,
+            hipLaunchKernelGGL(mr_zd_io(Mo), dim3((unsigned)mr_zd_grid(nt, Mo)), dim3(1024), 0, s,
                                fo.tws, A, S, out, plane, N, L, nc, coil0, cno, coil0 > 0 ? 1 : 0,
                                nt);
             MR_LAUNCH_CHECK("mr_k_io_dma");

@@ -634,12 +634,17 @@ constexpr int MR_EP_NST = 4;
 
 constexpr int mr_ep_lg(int v) { return v <= 1 ? 0 : 1 + mr_ep_lg(v / 2); }
 
-// The twiddle of each of a work-item's butterflies, for every stage of a
+// Twiddles of a stage, WN per butterfly: 1 and the stage forms the powers, or
+// all of them (WN >= R - 1).
+template <int WN> using mr_ep_tw = float2[MR_EP_KMAX][WN];
+
+// The twiddles of each of a work-item's butterflies, for every stage of a
 // tile of PT pencils: the same for every tile, so they are loaded once per
 // workgroup and no vector memory load (which completes in order) waits
-// behind the next tile's rows.
-template <int N, int S, int NT, int PT, class TW>
-__device__ __forceinline__ void mr_ep_twload(float2 (&w)[MR_EP_NST][MR_EP_KMAX], const TW &tw)
+// behind the next tile's rows. From 64 pencils on they are the same in a whole
+// wavefront and stay in scalar registers.
+template <int N, int S, int NT, int PT, int WN, class TW>
+__device__ __forceinline__ void mr_ep_twload(mr_ep_tw<WN> (&w)[MR_EP_NST], const TW &tw)
 {
     constexpr mr_ct_fac F = mr_ct_factor(N);
     static_assert(F.rest == 1 && F.nst <= MR_EP_NST, "length must be 2^a 3^b 5^c 7^d");
@@ -656,11 +661,20 @@ __device__ __forceinline__ void mr_ep_twload(float2 (&w)[MR_EP_NST][MR_EP_KMAX],
                 if (f < NB) {
                     const unsigned j = (unsigned)(f >> mr_ep_lg(PT));
                     const unsigned kk = j - mr_cdiv<NS>::q(j) * NS;
-                    w[S][k] = tw.get(NS + kk - 1, 0u);
+                    static_assert(WN == 1 || WN >= R - 1, "twiddles per butterfly");
+#pragma unroll
+                    for (int r = 0; r < (WN == 1 ? 1 : R - 1); ++r) {
+                        float2 t = tw.get((r + 1) * NS + kk - 1, 0u);
+                        if constexpr (PT >= 64) {
+                            t.x = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(t.x)));
+                            t.y = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(t.y)));
+                        }
+                        w[S][k][r] = t;
+                    }
                 }
             }
         }
-        mr_ep_twload<N, S + 1, NT, PT>(w, tw);
+        mr_ep_twload<N, S + 1, NT, PT, WN>(w, tw);
     }
 }
 
@@ -668,9 +682,8 @@ __device__ __forceinline__ void mr_ep_twload(float2 (&w)[MR_EP_NST][MR_EP_KMAX],
 // f mod PT and butterfly f / PT, so neighbouring lanes touch one row. OOP:
 // the inputs come from rd(pencil, element) instead of A, and no barrier
 // separates the reads from the writes.
-template <int N, int S, bool INV, int NT, int PT, bool OOP = false, class RD = int>
-__device__ __forceinline__ void mr_ep_stage(float2 *A, const float2 (&ws)[MR_EP_KMAX],
-                                            const RD &rd = 0)
+template <int N, int S, bool INV, int NT, int PT, bool OOP = false, int WN, class RD = int>
+__device__ __forceinline__ void mr_ep_stage(float2 *A, const mr_ep_tw<WN> &ws, const RD &rd = 0)
 {
     constexpr mr_ct_fac F = mr_ct_factor(N);
     constexpr int R = F.r[S], NS = F.ns[S];
@@ -701,10 +714,11 @@ __device__ __forceinline__ void mr_ep_stage(float2 *A, const float2 (&ws)[MR_EP_
             const unsigned jn = mr_cdiv<NS>::q((unsigned)j), kk = (unsigned)j - jn * NS;
             if constexpr (NS > 1) {
                 float2 wp[RW];
-                wp[0] = ws[k];
+                wp[0] = ws[k][0];
 #pragma unroll
                 for (int r = 1; r < R; ++r) {
-                    if (r >= 2) wp[r - 1] = cmul(wp[r / 2 - 1], wp[r - r / 2 - 1]);
+                    if constexpr (WN > 1) wp[r - 1] = ws[k][r - 1];
+                    else if (r >= 2) wp[r - 1] = cmul(wp[r / 2 - 1], wp[r - r / 2 - 1]);
                     v[k][r] = INV ? cmulc(wp[r - 1], v[k][r]) : cmul(wp[r - 1], v[k][r]);
                 }
             }
@@ -717,13 +731,13 @@ __device__ __forceinline__ void mr_ep_stage(float2 *A, const float2 (&ws)[MR_EP_
 }
 
 // Stages S .. last, in place.
-template <int N, int S, bool INV, int NT, int PT>
-__device__ __forceinline__ void mr_ep_fft(float2 *A, const float2 (&w)[MR_EP_NST][MR_EP_KMAX])
+template <int N, int S, bool INV, int NT, int PT, int WN>
+__device__ __forceinline__ void mr_ep_fft(float2 *A, const mr_ep_tw<WN> (&w)[MR_EP_NST])
 {
     constexpr mr_ct_fac F = mr_ct_factor(N);
     if constexpr (S < F.nst) {
-        mr_ep_stage<N, S, INV, NT, PT>(A, w[S]);
-        mr_ep_fft<N, S + 1, INV, NT, PT>(A, w);
+        mr_ep_stage<N, S, INV, NT, PT, false, WN>(A, w[S]);
+        mr_ep_fft<N, S + 1, INV, NT, PT, WN>(A, w);
     }
 }
 
@@ -740,8 +754,8 @@ mr_fft_axis_dma(const float2 *tws, Load ld, Store st, long long ntiles)
     // (and does not wait for them there).
     __shared__ __align__(16) float2 A[16 * N];
     __shared__ __align__(16) float2 B[16 * N];
-    float2 w[MR_EP_NST][MR_EP_KMAX];
-    mr_ep_twload<N, 0, NT, 16>(w, mr_tw_buf{mr_rsrc(tws, (unsigned)N * 8u)});
+    mr_ep_tw<1> w[MR_EP_NST];
+    mr_ep_twload<N, 0, NT, 16, 1>(w, mr_tw_buf{mr_rsrc(tws, (unsigned)N * 8u)});
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int ns = RW::rows(ld), c = RW::shift(ld);
