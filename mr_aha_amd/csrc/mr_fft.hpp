@@ -398,46 +398,111 @@ __device__ __forceinline__ void mr_stage(const V *__restrict__ A, V *__restrict_
     }
 }
 
-// Any radix: each thread evaluates one output of one butterfly as a length-R
-// dot product; the combined stage and DFT exponent is r (k + Ns q) stride,
-// looked up in the natural-order table tw (global memory).
-template <bool INV, typename V>
-__device__ __forceinline__ void mr_stage_any(const V *__restrict__ A, V *__restrict__ B,
-                                             const V *tw, int n, int ns, int tp, int Ns, int RR)
+// Stage of an odd radix RR without an unrolled butterfly (a prime from 11 on).
+// With the stage's twiddles in, s_r = x_r + x_{RR-r} and d_r = x_r - x_{RR-r}
+// (1 <= r <= h = (RR-1)/2, placed where x_r and x_{RR-r} were), outputs q and
+// RR - q are C -+ i D with
+//   C = x_0 + sum_r cos(2 pi q r / RR) s_r,  D = sum_r sin(2 pi q r / RR) d_r
+// (signs swapped for the inverse): a quarter of the multiplications of the sum
+// over all r for every q. A work-item computes QB outputs q, which share the
+// reads of s and d. tw: natural-order table in LDS, exp(-2 pi i e / n); the
+// divisions are one per work-item.
+template <int QB, bool INV, typename V>
+__device__ __forceinline__ void mr_stage_odd_sum(const V *__restrict__ A, V *__restrict__ B,
+                                                 const V *__restrict__ tw, int n, int ns, int tp,
+                                                 int Ns, int RR)
 {
-    const int m = n / RR;
-    const int stride = n / (Ns * RR);
-    const int per = m * RR;  // outputs per pencil
-    for (int f = threadIdx.x; f < tp * per; f += blockDim.x) {
-        const int p = f / per;
-        const int rem = f - p * per;
-        const int j = rem / RR;
-        const int q = rem - j * RR;
-        const int k = j % Ns;
+    using T = decltype(V::x);
+    const int m = n / RR, h = (RR - 1) / 2, ng = (h + QB) / QB, cols = tp * m;   // q = 0 .. h
+    for (int f = threadIdx.x; f < cols * ng; f += blockDim.x) {
+        const int g = f / cols, c = f - g * cols, j = c / tp, p = c - j * tp;
         const V *a = A + p * ns + j;
-        // exponent (k + Ns q) stride r mod n, stepped instead of divided
-        const int step = (int)((long long)(k + Ns * q) * stride % n);
-        int idx = 0;
-        V acc = cmake<V>(0, 0);
-        for (int r = 0; r < RR; ++r) {
-            const V w = tw[idx];
-            acc = cadd(acc, INV ? cmulc(w, a[r * m]) : cmul(w, a[r * m]));
-            idx += step;
-            if (idx >= n) idx -= n;
+        const V x0 = a[0];
+        V C[QB], D[QB];
+        int at[QB], step[QB];
+#pragma unroll
+        for (int i = 0; i < QB; ++i) {
+            const int q = g * QB + i <= h ? g * QB + i : h;
+            C[i] = x0;
+            D[i] = cmake<V>(0, 0);
+            at[i] = 0;
+            step[i] = q * m;   // 2 pi q / RR in units of 2 pi / n
         }
-        B[p * ns + (j / Ns) * Ns * RR + k + q * Ns] = acc;
+        const V *sp = a + m, *dp = a + (RR - 1) * m;
+        for (int r = 1; r <= h; ++r, sp += m, dp -= m) {
+            const V s = *sp, d = *dp;
+#pragma unroll
+            for (int i = 0; i < QB; ++i) {
+                at[i] += step[i];
+                if (at[i] >= n) at[i] -= n;
+                const V w = tw[at[i]];
+                const T cs = w.x, sn = -w.y;
+                C[i].x += cs * s.x;
+                C[i].y += cs * s.y;
+                D[i].x += sn * d.x;
+                D[i].y += sn * d.y;
+            }
+        }
+        const int jn = j / Ns;
+        V *b = B + p * ns + jn * Ns * RR + (j - jn * Ns);
+#pragma unroll
+        for (int i = 0; i < QB; ++i) {
+            const int q = g * QB + i;
+            if (q > h) break;
+            const T dx = INV ? -D[i].y : D[i].y, dy = INV ? D[i].x : -D[i].x;   // -+ i D
+            b[q * Ns] = cmake<V>(C[i].x + dx, C[i].y + dy);
+            if (q > 0) b[(RR - q) * Ns] = cmake<V>(C[i].x - dx, C[i].y - dy);
+        }
     }
 }
 
+// 112x131x34, L=6, 16 coils (262 along y) and 58x57x58, L=7, 15 coils (4 29, 6
+// 19, 4 29), whole apply, with one output per work-item, a sum over all r and
+// the table in global memory -> this: 25.1 -> 4.5 and 18.1 -> 5.6 ms; 2D 173x173,
+// L=8, 8 coils (346 both ways) 7.0 -> 0.54 ms.
+template <bool INV, typename V>
+__device__ __forceinline__ void mr_stage_odd(V *__restrict__ A, V *__restrict__ B,
+                                             const V *__restrict__ tw, int n, int ns, int tp,
+                                             int Ns, int RR)
+{
+    const int m = n / RR, h = (RR - 1) / 2, cols = tp * m, stride = m / Ns;
+    for (int f = threadIdx.x; f < cols * h; f += blockDim.x) {
+        const int r = f / cols, c = f - r * cols, j = c / tp, p = c - j * tp, k = j % Ns;
+        V *u = A + p * ns + j + (r + 1) * m, *v = A + p * ns + j + (RR - 1 - r) * m;
+        V x = *u, y = *v;
+        if (k > 0) {
+            const V wx = tw[k * (r + 1) * stride], wy = tw[k * (RR - 1 - r) * stride];
+            x = INV ? cmulc(wx, x) : cmul(wx, x);
+            y = INV ? cmulc(wy, y) : cmul(wy, y);
+        }
+        *u = cadd(x, y);
+        *v = cmake<V>(x.x - y.x, x.y - y.y);
+    }
+    __syncthreads();
+    // outputs per work-item: the width whose rounds of work-items cost least
+    // (QB products and two reads each)
+    auto cost = [&](int qb) {
+        const int items = cols * ((h + qb) / qb);
+        return (items + (int)blockDim.x - 1) / (int)blockDim.x * (qb + 1);
+    };
+    const int c3 = cost(3), c4 = cost(4), c6 = cost(6);
+    if (c6 <= c4 && c6 <= c3) mr_stage_odd_sum<6, INV, V>(A, B, tw, n, ns, tp, Ns, RR);
+    else if (c4 <= c3) mr_stage_odd_sum<4, INV, V>(A, B, tw, n, ns, tp, Ns, RR);
+    else mr_stage_odd_sum<3, INV, V>(A, B, tw, n, ns, tp, Ns, RR);
+}
+
 // Full transform of tp pencils held in LDS buffer A (B is scratch of the
-// same size). Returns the buffer that holds the result.
+// same size). Returns the buffer that holds the result. tw: LDS, n entries,
+// holding f.tws; the radices without an unrolled butterfly come last, and with
+// them f.tw takes its place.
 template <bool INV, typename R>
 __device__ typename cvec<R>::T *mr_fft_lds(const mr_fft_len<R> &f, typename cvec<R>::T *A,
-                                           typename cvec<R>::T *B, const typename cvec<R>::T *tw,
-                                           int ns, int tp)
+                                           typename cvec<R>::T *B, typename cvec<R>::T *tw, int ns,
+                                           int tp)
 {
     using V = typename cvec<R>::T;
     int Ns = 1;
+    bool natural = false;
     for (int s = 0; s < f.nst; ++s) {
         const int RR = f.radix[s];
         const mr_fdiv &md = f.mdiv[s], &nd = f.nsdiv[s];
@@ -450,7 +515,14 @@ __device__ typename cvec<R>::T *mr_fft_lds(const mr_fft_len<R> &f, typename cvec
         case 7: mr_stage<7, INV, V>(A, B, tw, f.n, ns, tp, Ns, md, nd); break;
         case 8: mr_stage<8, INV, V>(A, B, tw, f.n, ns, tp, Ns, md, nd); break;
         case 10: mr_stage<10, INV, V>(A, B, tw, f.n, ns, tp, Ns, md, nd); break;
-        default: mr_stage_any<INV, V>(A, B, f.tw, f.n, ns, tp, Ns, RR); break;
+        default:
+            if (!natural) {
+                natural = true;
+                for (int i = threadIdx.x; i < f.n; i += blockDim.x) tw[i] = f.tw[i];
+                __syncthreads();
+            }
+            mr_stage_odd<INV, V>(A, B, tw, f.n, ns, tp, Ns, RR);
+            break;
         }
         __syncthreads();
         V *t = A; A = B; B = t;
@@ -547,9 +619,12 @@ mr_fft_axis_kernel(mr_fft_len<R> f, Load ld, Store st, long long npencil, int lg
     V *acc = B0 + (size_t)TX * ns;
     const long long p0 = pbase + mr_xcd_block(blockIdx.x, gridDim.x) * TX;
     const int tp = (int)((npencil - p0 < TX) ? (npencil - p0) : TX);
-    for (int i = threadIdx.x; i < n; i += blockDim.x) tw[i] = f.tws[i];
+    const int last = f.nst > 0 ? f.radix[f.nst - 1] : 2;
+    const bool odd = last > 8 && last != 10;   // ends with f.tw in place of f.tws
     const int nsub = ld.nsub();
     for (int sub = 0; sub < nsub; ++sub) {
+        if (sub == 0 || odd)
+            for (int i = threadIdx.x; i < n; i += blockDim.x) tw[i] = f.tws[i];
         if (threadIdx.x < tp) {
             lpb[threadIdx.x] = ld.pencil(p0 + threadIdx.x, sub);
             spb[threadIdx.x] = st.pencil(p0 + threadIdx.x, sub);
