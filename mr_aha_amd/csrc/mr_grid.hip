@@ -361,9 +361,9 @@ int mr_grid_samples_build(const mr_grid &g, const float *traj, long long Ntrajs,
 // is even. A tile at the centre of radial samples has a thousand times the
 // candidates of one at the edge, and with one wavefront per tile the whole
 // pass waited for it. Measured, one wavefront per tile and now: 256x256 L=8
-// (512 x 512 samples, 36 sets) 2.58 -> 0.34 ms, 192x192x32 L=8 (1152 sets)
-// 26.9 -> 3.8 ms, of which the 10.9 GB of output take 2.0, 96^3 L=4 (4000 x
-// 192 samples) 49.7 -> 3.8 ms (9.1 GB, 1.7 ms); per sample, 128 x 384 samples
+// (512 x 512 samples, 36 sets) 2.58 -> 0.25 ms, 192x192x32 L=8 (1152 sets)
+// 26.9 -> 3.2 ms, of which the 10.9 GB of output take 2.0, 96^3 L=4 (4000 x
+// 192 samples) 49.7 -> 4.7 ms (9.1 GB, 1.7 ms); per sample, 128 x 384 samples
 // onto 384x384, 4 sets, 1.26 -> 0.09 ms.
 // ---------------------------------------------------------------------------
 
@@ -455,6 +455,9 @@ mr_k_spread(mr_grid g, const int *__restrict__ i0s, const int *__restrict__ rds,
                                                        __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
             double *ws = sh.w + slot * STR;
             sh.key[slot] = PER_SAMPLE ? i : rds[i];
+            // all loads before the first LDS write: one wait instead of one per value
+            // (256x256 L=8 0.33 -> 0.25 ms, 96^3 L=4 per chunk 1.84 -> 1.57)
+            double v[D][BS];
 #pragma unroll
             for (int a = 0; a < D; ++a) {
                 const double *wt = wts + ((long long)i * D + a) * w;
@@ -462,9 +465,11 @@ mr_k_spread(mr_grid g, const int *__restrict__ i0s, const int *__restrict__ rds,
                 for (int b = 0; b < BS; ++b) {
                     int o = o0[a] + b;
                     if (o >= g.nf[a]) o -= g.nf[a];
-                    ws[a * BS + b] = (o < w) ? wt[o] : 0.0;
+                    v[a][b] = (o < w) ? wt[o] : 0.0;
                 }
             }
+#pragma unroll
+            for (int a = 0; a < D * BS; ++a) ws[a] = v[a / BS][a % BS];
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();

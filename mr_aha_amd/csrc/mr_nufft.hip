@@ -14,7 +14,7 @@
 // first transform pass, cropping of the last ones, and the passes skip the
 // lines that are zero or not kept. 192x192 L=4, 4 coils, 128 x 384 samples:
 // apply
-// 876 -> 450 us, 238 us with the gridding's part (mr_grid.hip).
+// 876 -> 450 us, 222 us with the gridding's part (mr_grid.hip).
 
 #include "mr_grid.hpp"
 
