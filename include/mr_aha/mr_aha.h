@@ -238,7 +238,9 @@ MR_EXPORT int mr_op_info(mr_op op, mr_op_info_t *info);
 MR_EXPORT int mr_op_kernel(mr_op op, int k, const mr_complex **d_phi2_toep);
 /* Reference: mr_aha.h:1070. */
 MR_EXPORT int mr_op_destroy(mr_op op);
-/* Reference: mr_aha.h:1086. */
+/* After a device reset: releases the host side of the operator and touches no
+ * device memory. Abandon all operators of the device before any other call on
+ * it. Reference: mr_aha.h:1086. */
 MR_EXPORT int mr_op_abandon(mr_op op);
 
 /* Toeplitz kernel from Gram blocks and trajectory. Reference:

@@ -803,6 +803,10 @@ extern "C" MR_EXPORT int mr_aha_plan_destroy(mr_aha_plan plan)
     return MR_SUCCESS;
 }
 
+// The host side alone: after a device reset the plan's buffers and events are
+// gone, and their addresses may belong to someone else by now.
+void mr_aha_plan_abandon(mr_aha_plan plan) { delete plan; }
+
 int mr_bdt_launch(const mr_dims &d, float2 *K, const float2 *ker, const int *inv,
                   long long kstride, int nc, bool masked, hipStream_t s);
 bool mr_bdm_launch(const mr_dims &d, float2 *K, const float2 *ker, const int *inv,

@@ -444,6 +444,13 @@ size_t round256(size_t b) { return (b + 255) & ~size_t(255); }
 
 }  // namespace
 
+void mr_cg_forget(int dev)
+{
+    if (dev < 0 || dev >= MR_CG_MAX_DEVICES) return;
+    std::lock_guard<std::mutex> lk(g_scratch_mu);
+    g_scratch_ptr[dev] = nullptr;
+}
+
 extern "C" MR_EXPORT int mr_op_cg(mr_op op, mr_op op_refresh, const mr_complex *d_b,
                                   mr_complex *d_x, double lambda, int n_iter, int refresh,
                                   int flags, double *res_hist)

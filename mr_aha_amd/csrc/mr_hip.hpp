@@ -80,6 +80,15 @@ size_t mr_ws_idle_bytes(int dev);
 // memory runs out.
 hipError_t mr_dev_malloc(void **p, size_t bytes);
 
+// After a device reset nothing that was allocated on the device exists any more.
+// mr_device_forget drops what this library keeps there (scratch blocks, twiddle
+// tables, the address of the CG work array) without freeing or reusing it;
+// `since` is mr_device_epoch from before the caller's own allocations, so that
+// of all owners from before a reset only the first has an effect.
+unsigned mr_device_epoch(int dev);
+void mr_device_forget(int dev, unsigned since);
+void mr_cg_forget(int dev);
+
 // Budget = clamp(mem_fraction) * free bytes of the current device (idle
 // scratch counts as free).
 int mr_mem_budget(const mr_config *cfg, size_t *budget);

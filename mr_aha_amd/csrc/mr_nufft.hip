@@ -62,6 +62,9 @@ void mr_nufft_eng_destroy(mr_nufft_eng *e)
     if (e) mr_nufft_free(e);
 }
 
+// The host side alone (see mr_aha_plan_abandon).
+void mr_nufft_eng_abandon(mr_nufft_eng *e) { delete e; }
+
 int mr_nufft_eng_create(const mr_config *cfg, const mr_complex *d_phi2, const float *d_traj,
                         int64_t Ntrajs, int64_t Nkx, double upsampfac, mr_nufft_eng **out)
 {

@@ -32,6 +32,8 @@ int mr_nufft_eng_create(const mr_config *cfg, const mr_complex *d_phi2, const fl
 int mr_nufft_eng_execute(mr_nufft_eng *e, const mr_complex *d_x, const mr_complex *d_SEs,
                          mr_complex *d_out);
 void mr_nufft_eng_destroy(mr_nufft_eng *e);
+void mr_nufft_eng_abandon(mr_nufft_eng *e);
+void mr_aha_plan_abandon(mr_aha_plan plan);
 
 struct mr_op_s {
     mr_config cfg;
@@ -49,6 +51,7 @@ struct mr_op_s {
     unsigned *own_kq;   // 16-bit kernel entries (mr_op_set_kernel_format)
     float *own_ksc;     // and their block scales
     int kf;
+    unsigned epoch;     // mr_device_epoch of the primary device before its allocations
     mr_op_info_t info;
 };
 
@@ -166,6 +169,7 @@ static int mr_op_create_impl(const mr_config *cfg, const mr_op_inputs *in,
     p->opt = *o;
     p->opt.devices = nullptr;
     p->primary = primary;
+    p->epoch = mr_device_epoch(primary);
     p->stream = (hipStream_t)cfg->stream;
     if (hipSetDevice(primary) != hipSuccess || hipStreamSynchronize(p->stream) != hipSuccess) {
         mr_set_error("mr_op_create: HIP error on the primary device %d: %s", primary,
@@ -347,18 +351,17 @@ extern "C" MR_EXPORT int mr_op_destroy(mr_op op)
 }
 
 // After a device reset the operator's device memory no longer exists; only
-// the host side is released.
+// the host side is released. What the library keeps on the device between
+// calls (scratch, twiddle tables) died with it and is forgotten too, so that
+// no later call writes through it: abandon the operators of the device before
+// any other call on it.
 extern "C" MR_EXPORT int mr_op_abandon(mr_op op)
 {
     mr_clear_error();
     if (!op) return MR_SUCCESS;
-    if (op->plan) {
-        // The plan's buffers died with the context; release the host struct
-        // through the normal path, whose hipFree calls fail harmlessly.
-        mr_aha_plan_destroy(op->plan);
-    }
-    if (op->nu) mr_nufft_eng_destroy(op->nu);
-    (void)hipGetLastError();
+    mr_device_forget(op->primary, op->epoch);
+    if (op->plan) mr_aha_plan_abandon(op->plan);
+    if (op->nu) mr_nufft_eng_abandon(op->nu);
     delete op;
     return MR_SUCCESS;
 }

@@ -2,8 +2,10 @@
 // per-device cache of FFT twiddle tables.
 
 #include "mr_hip.hpp"
+#include "mr_scratch.hpp"
 
 #include <cmath>
+#include <iterator>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -97,117 +99,54 @@ void mr_fft_release_all()
 }
 
 // ---------------------------------------------------------------------------
-// Scratch blocks kept between calls (mr_hip.hpp). A block belongs to one
-// caller from mr_ws_get to mr_ws_put, so threads and streams never share one;
-// only the lists are guarded.
+// Scratch blocks kept between calls (mr_scratch.hpp, mr_hip.hpp)
 // ---------------------------------------------------------------------------
 namespace {
-struct ws_block {
-    void *p;
-    size_t bytes;
-    int dev;
-    unsigned long long tick;   // request count when it became idle
-};
-std::mutex g_ws_mu;
-std::vector<ws_block> g_ws_used, g_ws_idle;
-unsigned long long g_ws_tick = 0;
-
-// Return the idle blocks picked by `gone` to their devices (lock held).
-template <class F> bool ws_drop(F gone)
-{
-    int cur = -1;
-    (void)hipGetDevice(&cur);
-    bool any = false;
-    for (size_t i = 0; i < g_ws_idle.size();) {
-        if (!gone(g_ws_idle[i])) {
-            ++i;
-            continue;
-        }
-        const ws_block b = g_ws_idle[i];
-        g_ws_idle.erase(g_ws_idle.begin() + (long)i);
-        if (b.dev != cur) (void)hipSetDevice(b.dev);
-        (void)hipFree(b.p);
-        if (b.dev != cur) (void)hipSetDevice(cur);
-        any = true;
+struct ws_dev {
+    static int device()
+    {
+        int dev = -1;
+        return hipGetDevice(&dev) == hipSuccess ? dev : -1;
     }
-    return any;
-}
+    static void *alloc(size_t bytes)
+    {
+        void *p = nullptr;
+        if (hipMalloc(&p, bytes) == hipSuccess) return p;
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    static void release(int dev, void *p)
+    {
+        const int cur = device();
+        if (dev != cur) (void)hipSetDevice(dev);
+        (void)hipFree(p);
+        if (dev != cur) (void)hipSetDevice(cur);
+    }
+};
+mr_scratch<ws_dev> g_ws((size_t)MR_WS_MAX_IDLE, 64);
 }  // namespace
 
-size_t mr_ws_idle_bytes(int dev)
-{
-    std::lock_guard<std::mutex> lk(g_ws_mu);
-    size_t n = 0;
-    for (const ws_block &b : g_ws_idle) n += (b.dev == dev) ? b.bytes : 0;
-    return n;
-}
+size_t mr_ws_idle_bytes(int dev) { return g_ws.idle_bytes(dev); }
+void *mr_ws_get(size_t bytes) { return g_ws.get(bytes); }
+void mr_ws_put(void *p) { g_ws.put(p); }
 
 hipError_t mr_dev_malloc(void **p, size_t bytes)
 {
     hipError_t e = hipMalloc(p, bytes);
-    if (e == hipSuccess) return e;
-    int dev = -1;
-    (void)hipGetDevice(&dev);
-    bool any;
-    {
-        std::lock_guard<std::mutex> lk(g_ws_mu);
-        any = ws_drop([&](const ws_block &b) { return b.dev == dev; });
-    }
-    if (!any) return e;
+    if (e == hipSuccess || g_ws.release_idle(ws_dev::device()) == 0) return e;
     (void)hipGetLastError();
     return hipMalloc(p, bytes);
 }
 
-void *mr_ws_get(size_t bytes)
-{
-    if (bytes == 0) bytes = 1;
-    // whole megabytes above one, so that slightly different requests match
-    if (bytes > (1u << 20)) bytes = (bytes + (1u << 20) - 1) & ~(size_t)((1u << 20) - 1);
-    int dev = -1;
-    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-    {
-        std::lock_guard<std::mutex> lk(g_ws_mu);
-        ++g_ws_tick;
-        ws_drop([](const ws_block &b) { return g_ws_tick - b.tick > 64; });
-        size_t best = g_ws_idle.size();
-        for (size_t i = 0; i < g_ws_idle.size(); ++i) {
-            const ws_block &b = g_ws_idle[i];
-            if (b.dev == dev && b.bytes >= bytes && b.bytes <= 2 * bytes &&
-                (best == g_ws_idle.size() || b.bytes < g_ws_idle[best].bytes))
-                best = i;
-        }
-        if (best < g_ws_idle.size()) {
-            g_ws_used.push_back(g_ws_idle[best]);
-            g_ws_idle.erase(g_ws_idle.begin() + (long)best);
-            return g_ws_used.back().p;
-        }
-    }
-    void *p = nullptr;
-    if (mr_dev_malloc(&p, bytes) != hipSuccess) return nullptr;
-    std::lock_guard<std::mutex> lk(g_ws_mu);
-    g_ws_used.push_back(ws_block{p, bytes, dev, 0});
-    return p;
-}
+unsigned mr_device_epoch(int dev) { return g_ws.epoch(dev); }
 
-void mr_ws_put(void *p)
+void mr_device_forget(int dev, unsigned since)
 {
-    if (!p) return;
-    std::lock_guard<std::mutex> lk(g_ws_mu);
-    for (size_t i = 0; i < g_ws_used.size(); ++i) {
-        if (g_ws_used[i].p != p) continue;
-        g_ws_idle.push_back(g_ws_used[i]);
-        g_ws_idle.back().tick = g_ws_tick;
-        g_ws_used.erase(g_ws_used.begin() + (long)i);
-        break;
-    }
-    // over the limit: the blocks idle longest go first
-    size_t total = 0;
-    for (const ws_block &b : g_ws_idle) total += b.bytes;
-    while (total > (size_t)MR_WS_MAX_IDLE) {
-        const void *oldest = g_ws_idle.front().p;
-        total -= g_ws_idle.front().bytes;
-        ws_drop([&](const ws_block &b) { return b.p == oldest; });
-    }
+    if (!g_ws.forget(dev, since)) return;
+    mr_cg_forget(dev);
+    std::lock_guard<std::mutex> lk(g_tw_mu);
+    for (auto it = g_tw.begin(); it != g_tw.end();)
+        it = std::get<0>(it->first) == dev ? g_tw.erase(it) : std::next(it);
 }
 
 // ---------------------------------------------------------------------------
