@@ -7,7 +7,7 @@ gfx950 behind the reference's C ABI); this package only binds it.
 
 from ._lib import MRError, TrajType, Triangulation, backend, LIB_PATH  # noqa: F401
 from .api import (AhAOp, DEFAULT_MASK_RADIUS, MRConfig, aha_toeplitz, calc_mask,  # noqa: F401
-                  calc_toep, calc_toep_from_psf, create_op, make_config, num_tri,
-                  phi2_toep_shape)
+                  calc_toep, calc_toep_from_psf, create_op, idle_scratch, make_config, num_tri,
+                  phi2_toep_shape, release_scratch)
 
 __version__ = "1.0.0"

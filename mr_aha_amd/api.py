@@ -38,7 +38,8 @@ from ._lib import (CG_GRAPH, CG_ZERO_INIT, DEFAULT_MASK_RADIUS, KERNEL_BF16, KER
 
 __all__ = ["DEFAULT_MASK_RADIUS", "MRConfig", "MRError", "TrajType", "Triangulation",
            "make_config", "num_tri", "phi2_toep_shape", "calc_mask", "calc_toep",
-           "calc_toep_from_psf", "aha_toeplitz", "AhAOp", "create_op"]
+           "calc_toep_from_psf", "aha_toeplitz", "AhAOp", "create_op", "idle_scratch",
+           "release_scratch"]
 
 
 # ---------------------------------------------------------------------------
@@ -84,6 +85,41 @@ class _Arg:
         if handle is None:
             raise TypeError("stream must be None, an int handle or a torch.cuda.Stream")
         return int(handle) or None
+
+
+# ---------------------------------------------------------------------------
+# Device memory
+# ---------------------------------------------------------------------------
+
+def idle_scratch(device: int = -1) -> int:
+    """Bytes the library keeps idle on ``device`` (-1: the current one) for the
+    next kernel build (at most 4 GiB in a process). No counterpart in the
+    reference."""
+    n = ctypes.c_int64(0)
+    check(lib.mr_scratch_idle(int(device), ctypes.byref(n)), "mr_scratch_idle")
+    return int(n.value)
+
+
+def release_scratch(device: int = -1) -> int:
+    """Give that memory back to the device; returns the bytes. The library does
+    so itself when one of its own allocations fails; a program that allocates by
+    other means (torch) calls this when it needs the memory. No counterpart in
+    the reference."""
+    n = ctypes.c_int64(0)
+    check(lib.mr_scratch_release(int(device), ctypes.byref(n)), "mr_scratch_release")
+    return int(n.value)
+
+
+def _empty(shape, device, dtype=torch.complex64):
+    """An uninitialised array; idle scratch makes room for it when the device
+    is full."""
+    try:
+        return torch.empty(shape, dtype=dtype, device=device)
+    except torch.OutOfMemoryError:
+        index = torch.device(device).index
+        if release_scratch(-1 if index is None else index) == 0:
+            raise
+    return torch.empty(shape, dtype=dtype, device=device)
 
 
 # ---------------------------------------------------------------------------
@@ -238,7 +274,7 @@ def calc_mask(cfg: MRConfig, traj, radius: Optional[int] = None):
     if radius is not None:
         c.mask_radius = int(radius)
     ntr, nkx = _readouts(c, traj)
-    out = torch.empty(_size(lib.mr_pad_size, c), dtype=torch.int64, device=traj.device)
+    out = _empty(_size(lib.mr_pad_size, c), traj.device, torch.int64)
     count = ctypes.c_int64(0)
     check(lib.mr_calc_mask(ctypes.byref(c), _Arg.ptr(traj, "traj", "float32"), ntr, nkx,
                            _Arg.ptr(out, "mask", "int64"), ctypes.byref(count)), "mr_calc_mask")
@@ -249,7 +285,7 @@ def calc_toep(cfg: MRConfig, phi2, traj, mask=None, out=None):
     """Toeplitz kernel ``phi2_toep`` (reference: api.py:556-639)."""
     ntr, nkx = _gram_inputs(cfg, phi2, traj, mask)
     if out is None:
-        out = torch.empty(phi2_toep_shape(cfg), dtype=torch.complex64, device=phi2.device)
+        out = _empty(phi2_toep_shape(cfg), phi2.device)
     else:
         _Arg.numel(out, _size(lib.mr_phi2_toep_size, cfg), "out")
     check(lib.mr_calc_toep(ctypes.byref(cfg), _Arg.ptr(phi2, "phi2", "complex64"),
@@ -292,7 +328,7 @@ def aha_toeplitz(cfg: MRConfig, x, SEs, phi2_toep, mask=None, out=None):
 
 def _output_like(x, out):
     if out is None:
-        return torch.empty(x.shape, dtype=torch.complex64, device=x.device)
+        return _empty(x.shape, x.device)
     _Arg.numel(out, x.numel(), "out")
     return out
 
@@ -471,7 +507,7 @@ class AhAOp:
         """
         ptr = ctypes.c_void_p()
         check(lib.mr_op_kernel(self._open(), int(k), ctypes.byref(ptr)), "mr_op_kernel")
-        out = torch.empty(phi2_toep_shape(self._cfg), dtype=torch.complex64, device=self._device)
+        out = _empty(phi2_toep_shape(self._cfg), self._device)
         _memcpy_d2d(out.data_ptr(), ptr.value, out.numel() * 8)
         return out
 
@@ -517,7 +553,7 @@ class AhAOp:
             x = torch.complex(torch.randn(nx, generator=g), torch.randn(nx, generator=g))
             x = x.to(self._device)
         _Arg.numel(x, nx, "x")
-        out = torch.empty(x.shape, dtype=torch.complex64, device=x.device)
+        out = _empty(x.shape, x.device)
         torch.cuda.synchronize(self._device)   # x written on torch's stream is complete
         check(lib.mr_op_autotune(h, _Arg.ptr(x, "x", "complex64"),
                                  _Arg.ptr(out, "out", "complex64"), int(reps)), "mr_op_autotune")
@@ -553,7 +589,7 @@ class AhAOp:
         _Arg.numel(b, n, "b")
         flags = CG_GRAPH if graph else 0
         if x is None:
-            x = torch.empty(b.shape, dtype=torch.complex64, device=b.device)
+            x = _empty(b.shape, b.device)
             flags |= CG_ZERO_INIT
         else:
             _Arg.numel(x, n, "x")

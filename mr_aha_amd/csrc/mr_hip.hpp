@@ -71,7 +71,7 @@ void mr_pop_device(int prev);
 // caller alone, or null. mr_ws_put: hand it back once all work that uses it has
 // completed, whatever its stream. At most MR_WS_MAX_IDLE bytes stay idle in a
 // process; a block not used by 64 later requests, or any when an allocation of
-// this library fails, is returned to the device.
+// this library fails or mr_scratch_release is called, is returned to the device.
 #define MR_WS_MAX_IDLE (4LL << 30)
 void *mr_ws_get(size_t bytes);
 void mr_ws_put(void *p);

@@ -3,6 +3,7 @@
 
 #include "mr_hip.hpp"
 #include "mr_scratch.hpp"
+#include "mr_aha/mr_aha_scratch.h"
 
 #include <cmath>
 #include <iterator>
@@ -136,6 +137,22 @@ hipError_t mr_dev_malloc(void **p, size_t bytes)
     if (e == hipSuccess || g_ws.release_idle(ws_dev::device()) == 0) return e;
     (void)hipGetLastError();
     return hipMalloc(p, bytes);
+}
+
+extern "C" MR_EXPORT int mr_scratch_idle(int device, int64_t *bytes)
+{
+    mr_clear_error();
+    MR_REQUIRE(bytes != nullptr, "mr_scratch_idle: bytes is NULL");
+    *bytes = (int64_t)g_ws.idle_bytes(device < 0 ? ws_dev::device() : device);
+    return MR_SUCCESS;
+}
+
+extern "C" MR_EXPORT int mr_scratch_release(int device, int64_t *bytes)
+{
+    mr_clear_error();
+    const size_t n = g_ws.release_idle(device < 0 ? ws_dev::device() : device);
+    if (bytes) *bytes = (int64_t)n;
+    return MR_SUCCESS;
 }
 
 unsigned mr_device_epoch(int dev) { return g_ws.epoch(dev); }

@@ -21,7 +21,8 @@ public:
     // block goes back to the device
     mr_scratch(size_t max_idle, unsigned long long max_age) : max_idle_(max_idle), max_age_(max_age) {}
 
-    // A block of at least `bytes` on the current device, or null.
+    // A block of at least `bytes` (rounded up to megabytes, and up to an eighth
+    // more) on the current device, or null.
     void *get(size_t bytes)
     {
         if (bytes == 0) bytes = 1;
@@ -35,7 +36,7 @@ public:
             drop([&](const block &b) { return tick_ - b.tick > max_age_; });
             block *best = nullptr;
             for (block &b : blocks_)
-                if (b.idle && b.dev == dev && b.bytes >= bytes && b.bytes <= 2 * bytes &&
+                if (b.idle && b.dev == dev && b.bytes >= bytes && b.bytes - bytes <= bytes / 8 &&
                     (!best || b.bytes < best->bytes))
                     best = &b;
             if (best) {

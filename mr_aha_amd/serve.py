@@ -6,9 +6,11 @@ normal equations and its memory until it finishes. The server:
 
 * admits pending requests in arrival order while a slot is free and their
   HBM footprint (kernel, 16-bit copy, plan work buffers, the kernel build's
-  gridding chunks, CG vectors, maps; each an upper bound of what the library
+  scratch, CG vectors, maps; each an upper bound of what the library
   allocates for them) fits the remaining budget, so requests that arrive
-  while others run start as soon as memory and a slot free up;
+  while others run start as soon as memory and a slot free up; scratch that
+  finished builds left idle counts too, and is given back where it would keep
+  a request out;
 * runs every admitted request on its own non-blocking HIP stream from a
   worker thread (the library calls release the GIL), so kernel builds,
   applies and CG iterations of different requests overlap on the device;
@@ -91,7 +93,17 @@ def _build_component_bytes(req: Request) -> int:
 
 
 def build_bytes(req: Request) -> int:
-    return max(BUILD_BYTES, _build_component_bytes(req))
+    """Upper estimate of the kernel build's scratch: the gridding chunk, the
+    strengths of the Gram blocks, per sample its sort keys (twice), indexes
+    (twice), first points, readout and 16 weights an axis, and the sort's own
+    work; blocks may be an eighth larger than asked for, and whole megabytes."""
+    chunk = max(BUILD_BYTES, _build_component_bytes(req))
+    ntraj, nkx = int(req.traj.shape[-1]), int(req.traj.shape[-2])
+    planes = req.n_dim[2] if req.traj_type == "stack" else 1
+    strengths = req.L * (req.L + 1) // 2 * planes * ntraj * 16
+    axes = 3 if req.traj_type == "3D" else 2
+    samples = ntraj * nkx * (4 * 4 + 12 + 4 + axes * 16 * 8 + 16)
+    return (chunk + strengths + samples) * 9 // 8 + (32 << 20)
 
 
 def footprint_bytes(req: Request) -> int:
@@ -131,6 +143,17 @@ class Server:
         self._lock = threading.Condition()
         self._used = 0
         self._running = 0
+
+    def _fits(self, need: int) -> bool:
+        """Whether `need` more bytes fit the budget (lock held). Idle scratch of
+        finished builds is memory of its own; that of running ones lies within
+        their footprints as well, so what is given back here may be more than
+        it takes, never less."""
+        if self._running >= self.slots or self._used + need > self.budget:
+            return False
+        if self._used + need + api.idle_scratch() > self.budget:
+            api.release_scratch()
+        return True
 
     def _solve(self, req: Request, t0: float, ref_ev) -> None:
         # a non-blocking stream: the graph capture of one request must not be
@@ -212,7 +235,7 @@ class Server:
                     continue
                 need = footprint_bytes(head)
                 with self._lock:
-                    while self._running >= self.slots or self._used + need > self.budget:
+                    while not self._fits(need):
                         self._lock.wait(timeout=0.05)
                     self._used += need
                     self._running += 1

@@ -1,0 +1,59 @@
+"""Device memory that the library keeps or takes beside its arrays: the scratch
+of the kernel builds stays idle between them and goes back on request."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def mr():
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    import mr_aha_amd
+    return mr_aha_amd
+
+
+def _radial(tt, n, L, spokes, nkx, seed):
+    """Gram blocks and a radial trajectory on the device."""
+    rng = np.random.default_rng(seed)
+    nd = 3 if tt == "3D" else 2
+    d = rng.standard_normal((nd, spokes))
+    d /= np.sqrt((d ** 2).sum(0))
+    r = np.pi * (2.0 * np.arange(nkx) / nkx - 1.0)
+    planes = (n[2],) if tt == "stack" else ()
+    a = rng.standard_normal((L,) + planes + (spokes,)) + 1j * rng.standard_normal((L,) + planes + (spokes,))
+    up = lambda v: torch.from_numpy(np.ascontiguousarray(v)).cuda()  # noqa: E731
+    return (up((a[None] * np.conj(a[:, None])).astype(np.complex64)),
+            up((r[None, :, None] * d[:, None, :]).astype(np.float32)))
+
+
+def _free():
+    torch.cuda.synchronize()
+    return torch.cuda.mem_get_info()[0]
+
+
+def test_idle_scratch_goes_back(mr):
+    """Builds of two sizes leave at most 4 GiB idle; releasing returns exactly
+    that to the device, and the next builds equal the first."""
+    mr.release_scratch()
+    assert mr.idle_scratch() == 0
+    cases = [("2D", (160, 144), 6), ("stack", (64, 48, 12), 4)]
+    ins = [_radial(tt, n, L, 120, 200, 7 + i) for i, (tt, n, L) in enumerate(cases)]
+
+    def build():
+        return [mr.calc_toep(mr.make_config(tt, n, L), *ins[i]) for i, (tt, n, L) in enumerate(cases)]
+
+    first = build()
+    torch.cuda.empty_cache()
+    idle, free = mr.idle_scratch(), _free()
+    assert 0 < idle <= 4 << 30
+    assert mr.release_scratch() == idle
+    assert mr.idle_scratch() == 0 and mr.release_scratch() == 0
+    assert _free() - free >= idle
+    for a, b in zip(first, build()):
+        assert torch.equal(torch.view_as_real(a), torch.view_as_real(b))
+    assert mr.idle_scratch() == idle   # the same requests, so the same blocks

@@ -150,3 +150,117 @@ def test_a_second_reset(ws):
     ws.t_reset()
     assert ws.t_forget(0, again) == 1
     assert ws.t_live(ws.t_get(4 * MB)) == 1 and ws.t_bad() == 0
+
+
+def test_a_block_serves_requests_of_its_size(ws):
+    """Up to an eighth smaller, never less: what a caller is given stays near
+    what it asked for."""
+    a = ws.t_get(9 * MB)
+    ws.t_put(a)
+    assert ws.t_get(8 * MB) == a
+    ws.t_put(a)
+    small = ws.t_get(6 * MB)
+    assert small != a
+    assert ws.t_get(10 * MB) not in (a, small)
+    assert ws.t_idle(0) == 9 * MB
+
+
+def test_idle_bytes_stay_within_the_limit(ws):
+    held = [ws.t_get(24 * MB) for _ in range(4)]
+    for p in held:
+        ws.t_put(p)
+        assert ws.t_idle(0) <= 64 * MB
+    assert ws.t_idle(0) == 48 * MB and ws.t_nlive() == 2
+    assert [ws.t_live(p) for p in held] == [0, 0, 1, 1]   # the longest idle went first
+    big = ws.t_get(65 * MB)
+    ws.t_put(big)
+    assert ws.t_idle(0) <= 64 * MB and ws.t_live(big) == 0
+
+
+def test_unused_blocks_go_back(built):
+    built.t_open(64 * MB, 8)
+    a = built.t_get(8 * MB)
+    built.t_put(a)
+    for _ in range(8):
+        built.t_put(built.t_get(2 * MB))
+        assert built.t_live(a) == 1
+    built.t_put(built.t_get(2 * MB))
+    assert built.t_live(a) == 0 and built.t_idle(0) == 2 * MB
+
+
+def test_a_full_device_takes_idle_blocks_back(ws):
+    ws.t_put(ws.t_get(8 * MB))
+    ws.t_device(1)
+    other = ws.t_get(4 * MB)
+    ws.t_put(other)
+    ws.t_device(0)
+    ws.t_room(1 * MB)
+    p = ws.t_get(9 * MB)          # more than the idle block, less than both
+    assert p and ws.t_idle(0) == 0
+    assert ws.t_idle(1) == 4 * MB and ws.t_live(other) == 1
+    assert ws.t_get(1 * MB) is None
+    assert ws.t_bad() == 0
+
+
+def test_an_array_that_does_not_fit_takes_idle_scratch(monkeypatch):
+    """Arrays of the Python interface are torch's; when torch has no memory left
+    the idle scratch is given back and the allocation tried once more."""
+    torch = pytest.importorskip("torch")
+    from mr_aha_amd import api
+    real, calls = torch.empty, []
+
+    def empty(shape, **kw):
+        calls.append(tuple(shape))
+        if len(calls) == 1:
+            raise torch.OutOfMemoryError("out of memory")
+        return real(shape, **kw)
+
+    monkeypatch.setattr(torch, "empty", empty)
+    monkeypatch.setattr(api, "release_scratch", lambda device=-1: 8 * MB)
+    assert api._empty((2, 3), "cpu").shape == (2, 3) and len(calls) == 2
+    calls.clear()
+    monkeypatch.setattr(api, "release_scratch", lambda device=-1: 0)
+    with pytest.raises(torch.OutOfMemoryError):
+        api._empty((2, 3), "cpu")
+    assert len(calls) == 1
+
+
+def test_admission_counts_idle_scratch(monkeypatch):
+    """A request is admitted only when it, those running and the idle scratch
+    fit the budget together; the scratch makes room, the running ones do not."""
+    from mr_aha_amd import api, serve
+    idle = [6 * MB]
+    given = []
+
+    def release(device=-1):
+        given.append(idle[0])
+        idle[0] = 0
+        return given[-1]
+
+    monkeypatch.setattr(api, "idle_scratch", lambda device=-1: idle[0])
+    monkeypatch.setattr(api, "release_scratch", release)
+    srv = serve.Server(budget_bytes=16 * MB, slots=2)
+    assert srv._fits(10 * MB) and not given
+    assert srv._fits(11 * MB) and given == [6 * MB]
+    idle[0], srv._used, srv._running = 3 * MB, 8 * MB, 1
+    assert not srv._fits(9 * MB) and given == [6 * MB]
+    assert srv._fits(8 * MB) and given == [6 * MB, 3 * MB]
+    srv._running = 2
+    assert not srv._fits(1)
+
+
+def test_build_footprint_bounds_the_scratch():
+    """Every block that a build takes, by its formula: chunk, strengths, sample
+    tables (an eighth more each) and a megabyte for each of the dozen blocks."""
+    from types import SimpleNamespace
+    from mr_aha_amd import serve
+    for tt, n, L, ntr, nkx in [("2D", (320, 320), 16, 512, 640), ("stack", (256, 256, 48), 16, 400, 512),
+                               ("3D", (96, 96, 96), 4, 4000, 192), ("2D", (16, 16), 1, 1, 8)]:
+        req = SimpleNamespace(traj_type=tt, n_dim=n, L=L, precision="fp32", n_coils=4,
+                              traj=SimpleNamespace(shape=(3 if tt == "3D" else 2, nkx, ntr)))
+        m, d = ntr * nkx, 3 if tt == "3D" else 2
+        planes = n[2] if tt == "stack" else 1
+        blocks = [serve.BUILD_BYTES, L * (L + 1) // 2 * planes * ntr * 16, m * d * 16 * 8, 3 * m * 4]
+        blocks += [m * 4] * 5
+        assert serve.build_bytes(req) >= sum(b * 9 // 8 + MB for b in blocks)
+        assert serve.footprint_bytes(req) > serve.build_bytes(req)
