@@ -545,7 +545,7 @@ mr_k_spread(mr_grid g, const int *__restrict__ i0s, const int *__restrict__ rds,
 template <int D>
 __global__ void __launch_bounds__(64)
 mr_k_spread_sum(mr_grid g, const int2 *__restrict__ ext, long long next,
-                const double2 *__restrict__ part, double2 *__restrict__ fine)
+                const double2 *__restrict__ part, double2 *__restrict__ fine, int q0)
 {
     constexpr int BS = mr_spread_lds<D>::BS;
     const long long e0 = blockIdx.x;
@@ -560,8 +560,9 @@ mr_k_spread_sum(mr_grid g, const int2 *__restrict__ ext, long long next,
                          (long long)g.nf[0] * ((t[1] * BS + (lane / BS) % BS) +
                                                (long long)g.nf[1] *
                                                    (D == 3 ? t[2] * BS + lane / (BS * BS) : 0));
-    double2 *f = fine + (long long)blockIdx.y * g.nfine + gl;
-    const double2 *s = part + (long long)blockIdx.y * next * 64 + lane;
+    const long long q = q0 + (int)blockIdx.y;
+    double2 *f = fine + q * g.nfine + gl;
+    const double2 *s = part + q * next * 64 + lane;
     double2 a = *f;
 #pragma unroll 8
     for (long long e = e0; e < e1; ++e) {
@@ -597,9 +598,11 @@ static int mr_spread_launch(const mr_grid &g, const mr_grid_samples &s, const do
     }
 #undef MR_SPREAD
     MR_LAUNCH_CHECK("mr_k_spread");
-    if (s.next > 0) {
-        hipLaunchKernelGGL(mr_k_spread_sum<D>, dim3((unsigned)s.next, (unsigned)Q), dim3(64), 0,
-                           stream, g, s.ext, s.next, part, fine);
+    // a set per grid.y, of which a launch has 65535 at most
+    for (int y0 = 0; s.next > 0 && y0 < Q; y0 += 65535) {
+        hipLaunchKernelGGL(mr_k_spread_sum<D>,
+                           dim3((unsigned)s.next, (unsigned)std::min(Q - y0, 65535)), dim3(64), 0,
+                           stream, g, s.ext, s.next, part, fine, y0);
         MR_LAUNCH_CHECK("mr_k_spread_sum");
     }
     return MR_SUCCESS;
