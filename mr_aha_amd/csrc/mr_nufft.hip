@@ -48,12 +48,22 @@ struct mr_nufft_eng {
     mr_fft_len<double> fz;
 };
 
+// Buffers whose size goes with the coils per launch
+static void mr_nufft_free_batch(mr_nufft_eng *e)
+{
+    double2 **bufs[] = {&e->img, &e->acc, &e->fine, &e->tmp, &e->part};
+    for (double2 **p : bufs) {
+        if (*p) (void)hipFree(*p);
+        *p = nullptr;
+    }
+}
+
 static void mr_nufft_free(mr_nufft_eng *e)
 {
     mr_grid_samples_free(&e->smp, false);
     for (double *p : e->dc) if (p) (void)hipFree(p);
-    void *bufs[] = {e->phi2, e->img, e->acc, e->fine, e->tmp, e->part};
-    for (void *p : bufs) if (p) (void)hipFree(p);
+    if (e->phi2) (void)hipFree(e->phi2);
+    mr_nufft_free_batch(e);
     delete e;
 }
 
@@ -95,24 +105,35 @@ int mr_nufft_eng_create(const mr_config *cfg, const mr_complex *d_phi2, const fl
     const long long tmp = std::max(2 * Q * e->Mnu, Q * nhalf);
     const long long per = e->Nimg * cfg->L + Q * e->g.nfine + tmp + e->smp.part_elems(Q);
     // coils per launch: as many as fit MR_NU_BATCH_MB
-    // (MR_AHA_HIP_NU_MB overrides it), evened out; sets are
-    // counted in grid.y
-    long long nb = std::min<long long>(mr_env_ll("MR_AHA_HIP_NU_MB", MR_NU_BATCH_MB) * (1LL << 20) / (16 * per), 65535 / Q);
-    nb = std::max(1LL, std::min<long long>(nb, cfg->n_coils));
-    nb = mr_ceil_div(cfg->n_coils, mr_ceil_div(cfg->n_coils, nb));
-    e->nb = (int)nb;
+    // (MR_AHA_HIP_NU_MB overrides it) and the memory budget, evened out; sets are
+    // counted in grid.y. Fewer where the device has no room for them after all.
+    size_t budget = 0;
+    rc = mr_mem_budget(cfg, &budget);
+    if (rc != MR_SUCCESS) { mr_nufft_free(e); return rc; }
+    const long long most = std::min<long long>(mr_env_ll("MR_AHA_HIP_NU_MB", MR_NU_BATCH_MB) * (1LL << 20),
+                                               (long long)budget);
     const size_t img_bytes = (size_t)e->Nimg * cfg->L * sizeof(double2);
+    long long nb = std::min<long long>(most / (16 * per), 65535 / Q);
+    nb = std::max(1LL, std::min<long long>(nb, cfg->n_coils));
     hipError_t he = mr_dev_malloc((void **)&e->phi2, phi2_bytes);
-    if (he == hipSuccess) he = mr_dev_malloc((void **)&e->img, img_bytes * nb);
-    if (he == hipSuccess && nb < cfg->n_coils) he = mr_dev_malloc((void **)&e->acc, img_bytes);
-    if (he == hipSuccess)
-        he = mr_dev_malloc((void **)&e->fine, (size_t)(nb * Q * e->g.nfine) * sizeof(double2));
-    if (he == hipSuccess)
-        he = mr_dev_malloc((void **)&e->tmp, (size_t)(nb * tmp + MR_GRID_STR_PAD) * sizeof(double2));
+    for (; he == hipSuccess; nb /= 2) {
+        nb = mr_ceil_div(cfg->n_coils, mr_ceil_div(cfg->n_coils, nb));
+        e->nb = (int)nb;
+        he = mr_dev_malloc((void **)&e->img, img_bytes * nb);
+        if (he == hipSuccess && nb < cfg->n_coils) he = mr_dev_malloc((void **)&e->acc, img_bytes);
+        if (he == hipSuccess)
+            he = mr_dev_malloc((void **)&e->fine, (size_t)(nb * Q * e->g.nfine) * sizeof(double2));
+        if (he == hipSuccess)
+            he = mr_dev_malloc((void **)&e->tmp, (size_t)(nb * tmp + MR_GRID_STR_PAD) * sizeof(double2));
+        if (he == hipSuccess && e->smp.next > 0)
+            he = mr_dev_malloc((void **)&e->part, (size_t)e->smp.part_elems(nb * Q) * sizeof(double2));
+        if (he == hipSuccess || nb == 1) break;
+        (void)hipGetLastError();
+        mr_nufft_free_batch(e);
+        he = hipSuccess;
+    }
     e->k1 = e->tmp;
     e->k2 = e->tmp + nb * Q * e->Mnu;
-    if (he == hipSuccess && e->smp.next > 0)
-        he = mr_dev_malloc((void **)&e->part, (size_t)e->smp.part_elems(nb * Q) * sizeof(double2));
     if (he == hipSuccess) {
         rc = mr_grid_deconv(e->g, e->dc, e->s);
         if (rc != MR_SUCCESS) { mr_nufft_free(e); return rc; }

@@ -57,3 +57,37 @@ def test_idle_scratch_goes_back(mr):
     for a, b in zip(first, build()):
         assert torch.equal(torch.view_as_real(a), torch.view_as_real(b))
     assert mr.idle_scratch() == idle   # the same requests, so the same blocks
+
+
+def test_nufft_batches_within_the_budget(mr):
+    """The comparator's coils per launch follow mem_fraction: with a budget of a
+    few MB it takes one coil at a time (192x176, L=4: 15 MB a coil), in the
+    default one several, and both give the same result (the coils are summed in
+    the same order; 1e-6 for the interpolation's sums)."""
+    n, L, C = (192, 176), 4, 12
+    phi2, traj = _radial("2D", n, L, 40, 256, 3)
+    g = torch.Generator(device="cuda").manual_seed(9)
+    S = torch.randn((C,) + n[::-1], dtype=torch.complex64, device="cuda", generator=g)
+    x = torch.randn((L,) + n[::-1], dtype=torch.complex64, device="cuda", generator=g)
+    mr.release_scratch()
+    torch.cuda.empty_cache()
+
+    def create(fraction):
+        mr.release_scratch()
+        before = _free()
+        op = mr.create_op(mr.make_config("2D", n, L, n_coils=C, mem_fraction=fraction), S, phi2, traj,
+                          method="nufft")
+        mr.release_scratch()
+        return op, before - _free()
+
+    total = torch.cuda.mem_get_info()[1]
+    wide, wide_bytes = create(0.5)
+    with wide:
+        ref = wide(x)
+        torch.cuda.synchronize()
+    narrow, narrow_bytes = create(8e6 / total)
+    with narrow:
+        y = narrow(x)
+        assert float(torch.linalg.vector_norm(y - ref) / torch.linalg.vector_norm(ref)) < 1e-6
+    print(f"[nufft] {wide_bytes >> 20} MB in batches, {narrow_bytes >> 20} MB one at a time", flush=True)
+    assert wide_bytes > 6 * narrow_bytes
