@@ -11,14 +11,20 @@
 // Against the one-tile kernels, whose loads, transform and stores run one after
 // another, the bound moves towards memory. What decides is how many wavefronts
 // a CU holds: with 32-bit offsets from uniform bases, unmasked loads and the
-// work-item index hidden behind an empty asm, the kernels take 62 (y), 78 and 96
-// registers (outer) instead of 111 to 128 with spills, and the inverse outer
-// pass went from 3.93 to 2.05 ms at 256x256x48, L=16, 16 coils (6.9 GB). Before
+// work-item index hidden behind an empty asm, the kernels with 8 elements a
+// work-item take 62 (y), 78 and 96 registers (outer, forward and inverse)
+// instead of 111 to 128, and the inverse outer
+// pass went from 3.93 to 2.05 ms at 256x256x48, L=16, 16 coils (6.9 GB). With 12
+// elements (lengths 257 to 384) it is 78, 102 and 128, with the radices 11 and 13
+// 71, 87 and 106 (94, 118 and 128 with 12 elements); of these the forward outer
+// kernels keep 36 bytes of scratch a lane, the inverse one with 12 elements and a
+// radix 11 or 13 68 bytes. Before
 // -> now at that size: forward outer 3.62 -> 2.46, inverse 4.67 -> 2.05 ms;
 // 240x216x40, L=6, 10 coils: outer 0.59 + 0.75 -> 0.39 + 0.35 ms, y (432) 1.22 +
 // 1.20 -> 0.87 + 0.75 ms (3.0 GB each: 3.4 and 4.0 TB/s); an odd plane (143x134x54,
-// L=3, 6 coils, one pencil per workgroup before) 0.87 + 0.80 -> 0.07 + 0.07 ms. 
+// L=3, 6 coils, one pencil per workgroup before) 0.87 + 0.80 -> 0.07 + 0.07 ms.
 
+#include "mr_axis_form.hpp"
 #include "mr_axis_rt.hpp"
 #include "mr_xbd.hpp"
 #include "mr_fft_ct.hpp"
@@ -152,7 +158,7 @@ __device__ __forceinline__ void ax_st(float2 *base, unsigned off, float2 v)
 // a neighbour's (clamped) and puts zero in its place when the tile is written
 // to LDS.
 template <bool INV, int NT, int KE, int PT, bool BIG>
-__global__ void __launch_bounds__(NT, KE > 8 ? 5 : BIG ? 7 : 8)
+__global__ void __launch_bounds__(NT, ax_waves(AX_Y, KE, BIG))
 mr_k_axis_y(mr_rt_len f, const float2 *tws, mr_ax_y a, mr_fdiv idiv, int npencil, int nt)
 {
     constexpr int DE = NT / PT;
@@ -238,7 +244,7 @@ template <int PT> __device__ __forceinline__ ax_lane ax_lane_of(int lgxw)
 // = PT / XW coils, and takes ceil(nc / CW) rounds over the coils. Tiles run
 // over the ranks first, which share the rows of S.
 template <int NT, int KE, int PT, bool BIG>
-__global__ void __launch_bounds__(NT, KE > 8 ? 4 : BIG ? 5 : 6)
+__global__ void __launch_bounds__(NT, ax_waves(AX_FO, KE, BIG))
 mr_k_axis_fo(mr_rt_len f, const float2 *tws, mr_ax_z a, mr_fdiv ldiv, int lgxw, int nt)
 {
     constexpr int DE = NT / PT;
@@ -317,7 +323,7 @@ mr_k_axis_fo(mr_rt_len f, const float2 *tws, mr_ax_z a, mr_fdiv ldiv, int lgxw, 
 
 // N: a compiled length, or 0
 template <int NT, int KE, int PT, bool BIG, int N = 0>
-__global__ void __launch_bounds__(NT, KE > 8 ? 4 : BIG ? 4 : 5)
+__global__ void __launch_bounds__(NT, ax_waves(AX_IO, KE, BIG))
 mr_k_axis_io(mr_rt_len f, const float2 *tws, mr_ax_z a, mr_fdiv ldiv, int lgxw, int nt)
 {
     constexpr int DE = NT / PT;
@@ -414,30 +420,6 @@ mr_k_axis_io(mr_rt_len f, const float2 *tws, mr_ax_z a, mr_fdiv ldiv, int lgxw, 
     }
 }
 
-// Work-items, elements per work-item (the tile's registers) and pencils of a
-// tile of length n. Up to 256 every form keeps 8 elements and 16 pencils (whole
-// lines), so that short lengths do not leave lanes of a butterfly round idle. Up
-// to 384, 512 work-items with 12 elements: two workgroups per CU overlap their
-// phases, where 1024 with 8 leave one (320 along z of 160^3, L=8, 8 coils:
-// inverse 1.57 against 2.50 ms; 288 along y of 144^3: 1.34 against 1.66). Up to
-// 512 the y passes take 1024 work-items (432: 0.87 and 0.75 ms, 512 with 16
-// elements 0.89 and 0.78). The outer passes take 8 pencils there, and also below
-// when whole lines would give a CU fewer than two tiles (2D: 225x198, 396 along
-// y, inverse 40 us against 51 with 16 pencils). Beyond 512 the one-tile kernels
-// are as fast or faster (2D 640: inverse 56 us against 73).
-struct ax_form {
-    int nt, ke, pt;
-};
-ax_form ax_pick(int n, bool outer, bool few)
-{
-    if (n <= 64) return {128, 8, 16};
-    if (n <= 128) return {256, 8, 16};
-    if (n <= 256) return {512, 8, 16};
-    if (outer && (few || n > 384)) return {512, 8, 8};
-    if (n <= 384) return {512, 12, 16};
-    return {1024, 8, 16};
-}
-
 int ax_cus()
 {
     static const int n = [] {
@@ -464,20 +446,16 @@ bool ax_ok(const mr_fft_len<float> &f, mr_rt_len *rt, bool *big)
 }
 
 template <class K, class... Args>
-int ax_launch(K kernel, const ax_form &fm, int waves, int n, long long nt, hipStream_t s,
-              const char *name, Args... args)
+int ax_launch(K kernel, const ax_form &fm, ax_kind kind, bool big, int n, long long nt,
+              hipStream_t s, const char *name, Args... args)
 {
     const int NT = fm.nt;
-    const size_t lds = (size_t)n * (fm.pt + 1) * sizeof(float2);
+    const size_t lds = (size_t)ax_lds(fm, n);
     if (lds > 65536)
         MR_HIP_CHECK(hipFuncSetAttribute((const void *)kernel,
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    // wavefronts per CU by the kernel's registers, workgroups as the LDS allows
-    long long per = (long long)(163840 / lds);
-    const int most = waves * 64 / NT;
-    if (per > most) per = most;
-    if (per < 1) per = 1;
-    const long long grid = nt < ax_cus() * per ? nt : ax_cus() * per;
+    const long long most = (long long)ax_cus() * ax_per_cu(kind, fm, big, n);
+    const long long grid = nt < most ? nt : most;
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(NT), lds, s, args..., (int)nt);
     MR_LAUNCH_CHECK(name);
     return MR_SUCCESS;
@@ -493,12 +471,12 @@ int ax_launch(K kernel, const ax_form &fm, int waves, int n, long long nt, hipSt
     else if (fm.ke == 12) CALL(512, 12, 16);                                                     \
     else CALL(512, 8, 16);
 
-#define AX_Y1(INV, NT, KE, PT, BIG, W)                                                           \
-    ax_launch(mr_k_axis_y<INV, NT, KE, PT, BIG>, fm, W, f.n, nt, s, "mr_k_axis_y", rt, f.tws, a, \
-              idiv, (int)npencil)
-#define AX_Y(NT, KE, PT)                                                                         \
-    *rc = inverse ? (big ? AX_Y1(true, NT, KE, PT, true, 28) : AX_Y1(true, NT, KE, PT, false, 32)) \
-                  : (big ? AX_Y1(false, NT, KE, PT, true, 28) : AX_Y1(false, NT, KE, PT, false, 32))
+#define AX_Y1(INV, NT, KE, PT, BIG)                                                              \
+    ax_launch(mr_k_axis_y<INV, NT, KE, PT, BIG>, fm, AX_Y, BIG, f.n, nt, s, "mr_k_axis_y", rt,    \
+              f.tws, a, idiv, (int)npencil)
+#define AX_YF(NT, KE, PT)                                                                        \
+    *rc = inverse ? (big ? AX_Y1(true, NT, KE, PT, true) : AX_Y1(true, NT, KE, PT, false))        \
+                  : (big ? AX_Y1(false, NT, KE, PT, true) : AX_Y1(false, NT, KE, PT, false))
 
 bool mr_axis_rt_y(const mr_fft_len<float> &f, bool inverse, const mr_ax_y &a, long long npencil,
                   hipStream_t s, int *rc)
@@ -511,17 +489,17 @@ bool mr_axis_rt_y(const mr_fft_len<float> &f, bool inverse, const mr_ax_y &a, lo
     const mr_fdiv idiv = mr_fdiv_make((unsigned)a.I);
     const ax_form fm = ax_pick(f.n, false, false);
     const long long nt = mr_ceil_div(npencil, fm.pt);
-    AX_EACH(AX_Y)
+    AX_EACH(AX_YF)
     return true;
 }
 
-#define AX_Z1(K, NT, KE, PT, BIG, W)                                                             \
-    ax_launch(K<NT, KE, PT, BIG>, fm, W, f.n, nt, s, #K, rt, f.tws, a, ldiv, lgxw)
-#define AX_Z(NT, KE, PT)                                                                         \
-    *rc = inverse ? (big ? AX_Z1(mr_k_axis_io, NT, KE, PT, true, 16)                             \
-                         : AX_Z1(mr_k_axis_io, NT, KE, PT, false, 20))                           \
-                  : (big ? AX_Z1(mr_k_axis_fo, NT, KE, PT, true, 20)                             \
-                         : AX_Z1(mr_k_axis_fo, NT, KE, PT, false, 24))
+#define AX_Z1(K, KIND, NT, KE, PT, BIG)                                                          \
+    ax_launch(K<NT, KE, PT, BIG>, fm, KIND, BIG, f.n, nt, s, #K, rt, f.tws, a, ldiv, lgxw)
+#define AX_ZF(NT, KE, PT)                                                                        \
+    *rc = inverse ? (big ? AX_Z1(mr_k_axis_io, AX_IO, NT, KE, PT, true)                          \
+                         : AX_Z1(mr_k_axis_io, AX_IO, NT, KE, PT, false))                        \
+                  : (big ? AX_Z1(mr_k_axis_fo, AX_FO, NT, KE, PT, true)                          \
+                         : AX_Z1(mr_k_axis_fo, AX_FO, NT, KE, PT, false))
 
 bool mr_axis_rt_z(const mr_fft_len<float> &f, bool inverse, const mr_ax_z &a, hipStream_t s,
                   int *rc)
@@ -547,8 +525,8 @@ bool mr_axis_rt_z(const mr_fft_len<float> &f, bool inverse, const mr_ax_z &a, hi
         switch (f.n * 100 + fm.pt) {
 #define AX_ZN(N, NT, KE, PT)                                                                     \
     case N * 100 + PT:                                                                           \
-        *rc = ax_launch(mr_k_axis_io<NT, KE, PT, false, N>, fm, 20, f.n, nt, s, "mr_k_axis_io",   \
-                        rt, f.tws, a, ldiv, lgxw);                                               \
+        *rc = ax_launch(mr_k_axis_io<NT, KE, PT, false, N>, fm, AX_IO, false, f.n, nt, s,          \
+                        "mr_k_axis_io", rt, f.tws, a, ldiv, lgxw);                               \
         return true;
             AX_ZN(256, 512, 8, 16) AX_ZN(320, 512, 8, 8) AX_ZN(320, 512, 12, 16)
             AX_ZN(384, 512, 8, 8) AX_ZN(384, 512, 12, 16) AX_ZN(512, 512, 8, 8)
@@ -556,6 +534,6 @@ bool mr_axis_rt_z(const mr_fft_len<float> &f, bool inverse, const mr_ax_z &a, hi
         default: break;
         }
     }
-    AX_EACH(AX_Z)
+    AX_EACH(AX_ZF)
     return true;
 }
