@@ -563,7 +563,8 @@ class AhAOp:
     def tiles(self) -> dict:
         """Tiling in use (library entry mr_op_tiles): pencils per workgroup
         requested for the outer-axis, y, inverse y and inverse outer-axis FFT
-        passes (0: the built-in rule), whether the fused x pass runs
+        passes (0: the built-in rule; after `autotune`, for a pass on a
+        persistent kernel, the pencils of that kernel's own tile), whether the fused x pass runs
         two-coil workgroups and whether its block step runs on the matrix
         cores."""
         t = (ctypes.c_int * 6)()

@@ -437,6 +437,9 @@ struct mr_aha_plan_s {
     int rt_nt;
     int xbd_nt;           // its workgroup size
     int tile[4];          // pencils per workgroup of Fo, Fy, Iy, Io (0: default rule)
+    int fixed[4];         // pencils of a tile in the last execute where the pass ran on a
+                          // persistent kernel, which has its own width; else 0
+    bool tuned;           // mr_aha_plan_autotune has run
     int no_wide;          // 1: no two-coil 1024-thread fused workgroups
     mr_xbd_ct_fn xbd_mf;  // xbd_ct with the block step on the matrix cores, or null
     mr_xbd_ct_fn xbd_pd;  // persistent form of xbd_ct (one workgroup per CU), or null
@@ -1131,19 +1134,21 @@ static int mr_execute_xlast(mr_aha_plan p, const float2 *x, const float2 *S, con
         mr_zmap zm{V, lgT};
         mr_ld_sx_z ld{x, S, zm, plane, N, No, Mo, cno, L, coil0};
         mr_st_z st{A, zm, plane, Mo};
-        // pencils per workgroup: the autotuned width, else 2^lgT up to 64;
-        // MR_AHA_HIP_FO_TX overrides both, and likewise for the other passes
-        // below
+        // pencils per workgroup of the one-tile kernels: the autotuned width,
+        // else 2^lgT up to 64; MR_AHA_HIP_FO_TX overrides both, and likewise for
+        // the other passes below
         const int txo = (int)mr_env_ll("MR_AHA_HIP_FO_TX", p->tile[0] > 0 ? p->tile[0] : 1 << lgT);
         if (!two && mr_zd_ok(d, L, plane, x, S, A)) {
             const long long nt = (plane / 16) * (L / MR_ZD_LB);
             hipLaunchKernelGGL(mr_zd_fo(Mo), dim3((unsigned)mr_zd_grid(nt, Mo)), dim3(1024), 0, s,
                                fo.tws, x, S, A, plane, N, L, nc, coil0, cno, nt);
             MR_LAUNCH_CHECK("mr_k_fo_dma");
+            p->fixed[0] = MR_ZD_PT;
         } else {
             int rc = MR_SUCCESS;
             const mr_ax_z az{x, S, A, nullptr, plane, N, No, cno, L, nc, coil0, 0};
-            if (mr_outer_rt(Mo, false, plane) && mr_axis_rt_z(fo, false, az, s, &rc))
+            p->fixed[0] = mr_outer_rt(Mo, false, plane) ? mr_axis_rt_z(fo, false, az, s, &rc) : 0;
+            if (p->fixed[0])
                 MR_TRY(rc);
             else
                 MR_TRY((mr_fft_pass_ct<false>(fo, ld, st, plane * V, 0, txo, s, "Fo")));
@@ -1154,7 +1159,8 @@ static int mr_execute_xlast(mr_aha_plan p, const float2 *x, const float2 *S, con
         mr_ld_pad<float2, false> ld{A, Nx, My, Ny, d.c_n[1]};
         mr_st_axis<float2, false> st{B, Nx, My};
         const int txy = (int)mr_env_ll("MR_AHA_HIP_FY_TX", p->tile[1] > 0 ? p->tile[1] : 16);
-        MR_TRY((mr_fft_pass_ct<false>(p->fy, ld, st, (long long)Nx * Mz * V, 0, txy, s, "Fy")));
+        MR_TRY((mr_fft_pass_ct<false>(p->fy, ld, st, (long long)Nx * Mz * V, 0, txy, s, "Fy",
+                                      &p->fixed[1])));
         MR_TRY(mr_prof_mark(p, MR_ST_F2));
     }
     {
@@ -1192,7 +1198,8 @@ static int mr_execute_xlast(mr_aha_plan p, const float2 *x, const float2 *S, con
         mr_ld_axis<float2, false> ld{B, Nx, My};
         mr_st_crop<float2, false> st{A, Nx, My, Ny, d.c_n[1]};
         const int txy = (int)mr_env_ll("MR_AHA_HIP_IY_TX", p->tile[2] > 0 ? p->tile[2] : 16);
-        MR_TRY((mr_fft_pass_ct<true>(p->fy, ld, st, (long long)Nx * Mz * V, 0, txy, s, "Iy")));
+        MR_TRY((mr_fft_pass_ct<true>(p->fy, ld, st, (long long)Nx * Mz * V, 0, txy, s, "Iy",
+                                     &p->fixed[2])));
         MR_TRY(mr_prof_mark(p, MR_ST_I2));
     }
     {
@@ -1208,10 +1215,12 @@ static int mr_execute_xlast(mr_aha_plan p, const float2 *x, const float2 *S, con
                                fo.tws, A, S, out, plane, N, L, nc, coil0, cno, coil0 > 0 ? 1 : 0,
                                nt);
             MR_LAUNCH_CHECK("mr_k_io_dma");
+            p->fixed[3] = MR_ZD_PT;
         } else {
             int rc = MR_SUCCESS;
             const mr_ax_z az{nullptr, S, A, out, plane, N, No, cno, L, nc, coil0, coil0 > 0 ? 1 : 0};
-            if (mr_outer_rt(Mo, true, plane) && mr_axis_rt_z(fo, true, az, s, &rc))
+            p->fixed[3] = mr_outer_rt(Mo, true, plane) ? mr_axis_rt_z(fo, true, az, s, &rc) : 0;
+            if (p->fixed[3])
                 MR_TRY(rc);
             else
                 MR_TRY((mr_fft_pass_ct<true>(fo, ld, st, plane * L, (size_t)No, txi, s, "Io")));
@@ -1393,8 +1402,10 @@ extern "C" MR_EXPORT int mr_aha_plan_execute(mr_aha_plan plan, const mr_complex 
 }
 
 // Autotuner of the fused route: for each axis pass (Fo, Fy, Iy, Io; 2D: Fo,
-// Io) the tile widths 1..64 pencils are timed in turn on the caller's data
-// (`reps` applies each, HIP events per stage) and the fastest is kept; then
+// Io) on the one-tile kernels the tile widths 1..64 pencils are timed in turn on
+// the caller's data (`reps` applies each, HIP events per stage) and the fastest
+// is kept (the persistent kernels have a tile of their own, which no width
+// changes); then
 // the fused x pass's two-coil wide form against one coil per workgroup.
 // Every candidate computes the same arithmetic per pencil, so results do not
 // depend on the choice. The per-stage profile totals are cleared.
@@ -1426,6 +1437,7 @@ static int mr_autotune_impl(mr_aha_plan p, const mr_complex *x, const mr_complex
     for (int k = 0; k < 4 && rc == MR_SUCCESS; ++k) {
         const int t = idx[k];
         if (two && (t == 1 || t == 2)) continue;  // 2D: no separate y passes
+        if (p->fixed[t] > 0) continue;            // the width would change nothing
         int best = p->tile[t];
         double best_ms = 1e30;
         for (int cand = 1; cand <= 64 && rc == MR_SUCCESS; cand *= 2) {
@@ -1464,6 +1476,7 @@ static int mr_autotune_impl(mr_aha_plan p, const mr_complex *x, const mr_complex
         }
     }
     p->tuning = false;
+    p->tuned = rc == MR_SUCCESS;
     const int rc2 = zero_prof();
     return rc != MR_SUCCESS ? rc : rc2;
 }
@@ -1495,7 +1508,10 @@ extern "C" MR_EXPORT int mr_aha_plan_tiles(mr_aha_plan plan, int *tiles, int n)
     mr_clear_error();
     MR_REQUIRE(plan != nullptr, "mr_aha_plan_tiles: plan is NULL");
     MR_REQUIRE(tiles != nullptr || n == 0, "mr_aha_plan_tiles: tiles is NULL");
-    const int v[6] = {plan->tile[0], plan->tile[1], plan->tile[2], plan->tile[3],
+    int t[4];
+    for (int i = 0; i < 4; ++i)
+        t[i] = plan->tuned && plan->fixed[i] > 0 ? plan->fixed[i] : plan->tile[i];
+    const int v[6] = {t[0], t[1], t[2], t[3],
                       plan->xbd_nt > MR_XBD_THREADS ? 1 : 0,
                       (plan->xbd_mf && !plan->no_mf) ? 1 : 0};
     for (int i = 0; i < n && i < 6; ++i) tiles[i] = v[i];

@@ -478,19 +478,19 @@ int ax_launch(K kernel, const ax_form &fm, ax_kind kind, bool big, int n, long l
     *rc = inverse ? (big ? AX_Y1(true, NT, KE, PT, true) : AX_Y1(true, NT, KE, PT, false))        \
                   : (big ? AX_Y1(false, NT, KE, PT, true) : AX_Y1(false, NT, KE, PT, false))
 
-bool mr_axis_rt_y(const mr_fft_len<float> &f, bool inverse, const mr_ax_y &a, long long npencil,
+int mr_axis_rt_y(const mr_fft_len<float> &f, bool inverse, const mr_ax_y &a, long long npencil,
                   hipStream_t s, int *rc)
 {
     mr_rt_len rt;
     bool big;
-    if (!ax_ok(f, &rt, &big)) return false;
+    if (!ax_ok(f, &rt, &big)) return 0;
     // 32-bit pencil numbers and byte offsets within a tile's columns
-    if (npencil >= 0x7fffff00LL || a.I * 8 * (f.n + 1) * 17 >= 0xffffffffLL) return false;
+    if (npencil >= 0x7fffff00LL || a.I * 8 * (f.n + 1) * 17 >= 0xffffffffLL) return 0;
     const mr_fdiv idiv = mr_fdiv_make((unsigned)a.I);
     const ax_form fm = ax_pick(f.n, false, false);
     const long long nt = mr_ceil_div(npencil, fm.pt);
     AX_EACH(AX_YF)
-    return true;
+    return fm.pt;
 }
 
 #define AX_Z1(K, KIND, NT, KE, PT, BIG)                                                          \
@@ -501,12 +501,11 @@ bool mr_axis_rt_y(const mr_fft_len<float> &f, bool inverse, const mr_ax_y &a, lo
                   : (big ? AX_Z1(mr_k_axis_fo, AX_FO, NT, KE, PT, true)                          \
                          : AX_Z1(mr_k_axis_fo, AX_FO, NT, KE, PT, false))
 
-bool mr_axis_rt_z(const mr_fft_len<float> &f, bool inverse, const mr_ax_z &a, hipStream_t s,
-                  int *rc)
+int mr_axis_rt_z(const mr_fft_len<float> &f, bool inverse, const mr_ax_z &a, hipStream_t s, int *rc)
 {
     mr_rt_len rt;
     bool big;
-    if (!ax_ok(f, &rt, &big)) return false;
+    if (!ax_ok(f, &rt, &big)) return 0;
     // whole lines (16 positions) where that gives every CU two tiles, else
     // narrower tiles that take several coils at once
     const ax_form fm = ax_pick(f.n, true, mr_ceil_div(a.plane, 16) * a.L < 2 * ax_cus());
@@ -519,7 +518,7 @@ bool mr_axis_rt_z(const mr_fft_len<float> &f, bool inverse, const mr_ax_z &a, hi
     const long long cw = fm.pt >> lgxw;
     if (nt >= 0x7fffff00LL || a.plane * 8 * (f.n + 1) * (1 + (cw - 1) * a.L) >= 0xffffffffLL ||
         a.N * 8 * cw >= 0xffffffffLL)
-        return false;
+        return 0;
     const mr_fdiv ldiv = mr_fdiv_make((unsigned)a.L);
     if (inverse) {
         switch (f.n * 100 + fm.pt) {
@@ -527,7 +526,7 @@ bool mr_axis_rt_z(const mr_fft_len<float> &f, bool inverse, const mr_ax_z &a, hi
     case N * 100 + PT:                                                                           \
         *rc = ax_launch(mr_k_axis_io<NT, KE, PT, false, N>, fm, AX_IO, false, f.n, nt, s,          \
                         "mr_k_axis_io", rt, f.tws, a, ldiv, lgxw);                               \
-        return true;
+        return fm.pt;
             AX_ZN(256, 512, 8, 16) AX_ZN(320, 512, 8, 8) AX_ZN(320, 512, 12, 16)
             AX_ZN(384, 512, 8, 8) AX_ZN(384, 512, 12, 16) AX_ZN(512, 512, 8, 8)
 #undef AX_ZN
@@ -535,5 +534,5 @@ bool mr_axis_rt_z(const mr_fft_len<float> &f, bool inverse, const mr_ax_z &a, hi
         }
     }
     AX_EACH(AX_ZF)
-    return true;
+    return fm.pt;
 }

@@ -32,8 +32,9 @@ struct mr_ax_z {
     int nz, cz, L, nc, coil0, accumulate;
 };
 
-// Launch the pass, or return false when the length is not one of these (or
-// MR_AHA_HIP_AXRT=0). *rc receives the status of a launched pass.
-bool mr_axis_rt_y(const mr_fft_len<float> &f, bool inverse, const mr_ax_y &a, long long npencil,
+// Launch the pass and return the pencils of its tiles, or return 0 when the
+// length is not one of these (or MR_AHA_HIP_AXRT=0). *rc receives the status of
+// a launched pass.
+int mr_axis_rt_y(const mr_fft_len<float> &f, bool inverse, const mr_ax_y &a, long long npencil,
                   hipStream_t s, int *rc);
-bool mr_axis_rt_z(const mr_fft_len<float> &f, bool inverse, const mr_ax_z &a, hipStream_t s, int *rc);
+int mr_axis_rt_z(const mr_fft_len<float> &f, bool inverse, const mr_ax_z &a, hipStream_t s, int *rc);

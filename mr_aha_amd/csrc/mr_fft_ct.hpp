@@ -940,10 +940,14 @@ template <> struct mr_ax_dst<mr_st_crop<float2, false>> {
 // FP32 axis pass: the compile-time kernel for lengths 56, 256, 320, 384, 512
 // and 640 (MR_AHA_HIP_FFT_CT=0 turns it off); y passes of other lengths on the
 // run-time-length kernels (mr_axis_rt.hpp) where they can, mr_fft_pass otherwise.
+// *fixed (optional): the pencils of a tile where the kernel has its own width and
+// want_tx does not count, else 0.
 template <bool INV, class Load, class Store>
 int mr_fft_pass_ct(const mr_fft_len<float> &f, const Load &ld, const Store &st, long long npencil,
-                   size_t acc_per_pencil, int want_tx, hipStream_t stream, const char *name)
+                   size_t acc_per_pencil, int want_tx, hipStream_t stream, const char *name,
+                   int *fixed = nullptr)
 {
+    if (fixed) *fixed = 0;
     if (mr_env_ll("MR_AHA_HIP_FFT_CT", 1) != 0) {
         switch (f.n) {
 #define MR_CT_LEN(n)                                                                             \
@@ -959,7 +963,9 @@ int mr_fft_pass_ct(const mr_fft_len<float> &f, const Load &ld, const Store &st, 
         mr_ax_src<Load>::fill(a, ld);
         mr_ax_dst<Store>::fill(a, st);
         int rc = MR_SUCCESS;
-        if (npencil > 0 && mr_axis_rt_y(f, INV, a, npencil, stream, &rc)) return rc;
+        const int pt = npencil > 0 ? mr_axis_rt_y(f, INV, a, npencil, stream, &rc) : 0;
+        if (fixed) *fixed = pt;
+        if (pt) return rc;
     }
     return mr_fft_pass<float, INV>(f, ld, st, npencil, acc_per_pencil, want_tx, stream, name);
 }
