@@ -463,10 +463,16 @@ int ax_launch(K kernel, const ax_form &fm, ax_kind kind, bool big, int n, long l
 
 }  // namespace
 
-#define AX_EACH(CALL)                                                                            \
+// The forms of ax_pick: the narrow one is for outer passes, the wide one for y
+#define AX_EACH_Y(CALL)                                                                          \
     if (fm.nt == 128) CALL(128, 8, 16);                                                          \
     else if (fm.nt == 256) CALL(256, 8, 16);                                                     \
     else if (fm.nt == 1024) CALL(1024, 8, 16);                                                   \
+    else if (fm.ke == 12) CALL(512, 12, 16);                                                     \
+    else CALL(512, 8, 16);
+#define AX_EACH_Z(CALL)                                                                          \
+    if (fm.nt == 128) CALL(128, 8, 16);                                                          \
+    else if (fm.nt == 256) CALL(256, 8, 16);                                                     \
     else if (fm.pt == 8) CALL(512, 8, 8);                                                        \
     else if (fm.ke == 12) CALL(512, 12, 16);                                                     \
     else CALL(512, 8, 16);
@@ -489,7 +495,7 @@ int mr_axis_rt_y(const mr_fft_len<float> &f, bool inverse, const mr_ax_y &a, lon
     const mr_fdiv idiv = mr_fdiv_make((unsigned)a.I);
     const ax_form fm = ax_pick(f.n, false, false);
     const long long nt = mr_ceil_div(npencil, fm.pt);
-    AX_EACH(AX_YF)
+    AX_EACH_Y(AX_YF)
     return fm.pt;
 }
 
@@ -533,6 +539,6 @@ int mr_axis_rt_z(const mr_fft_len<float> &f, bool inverse, const mr_ax_z &a, hip
         default: break;
         }
     }
-    AX_EACH(AX_ZF)
+    AX_EACH_Z(AX_ZF)
     return fm.pt;
 }

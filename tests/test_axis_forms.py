@@ -99,3 +99,10 @@ def test_no_more_workgroups_than_a_cu_holds(forms, kernels):
                 held = 4 * occ * 64 // nt if nt < 256 else occ // (nt // 256)
                 assert per <= held, (kind, n, (nt, ke, pt), big, length, per, held)
         assert per == 1 or per * n * (pt + 1) * 8 <= 160 * 1024, (kind, n)
+
+
+def test_every_kernel_is_launched_by_some_length(forms, kernels):
+    used = {(kind, *form, big) for kind, _, _, _, big, form in _cases(forms)}
+    for kind, nt, ke, pt, big, length in kernels:
+        assert (kind, nt, ke, pt, big) in used, (kind, nt, ke, pt, big)
+        assert length <= NMAX
