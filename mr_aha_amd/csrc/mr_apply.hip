@@ -546,13 +546,17 @@ static void mr_plan_free_buffers(mr_aha_plan p)
 // Coils per workgroup of the run-time-length fused pass, `per` bytes of LDS a
 // coil: as many as keep two workgroups per CU (80 KB), rounded down to coil
 // pairs, which load each kernel entry once for both, and evened out over the
-// groups; else the pair in one workgroup of 1024 (160 KB), else one coil.
+// groups; else the pair in one workgroup of 1024 up to 128 KB, else one coil in 512
+// (the two workgroups of a CU overlap their phases). Pairs of up to 160 KB were
+// faster in some shapes and slower in others: fused pass, one coil -> pair,
+// 300x280x8 L=16 4 coils 2041 -> 1904 us, 320x280x8 L=14 6 coils 1917 -> 1873, 2D
+// 320x320 L=15 6 coils 327 -> 332, 270x200x8 L=16 5 coils 1580 -> 1641.
 // Where that leaves fewer than two workgroups per CU, smaller groups (a pair at
 // least): the rows are too few to fill the chip.
 static long long mr_xbd_rt_group(size_t per, int ncoil, long long rows)
 {
     long long g = (long long)(81920 / per);
-    if (g < 2) return (2 * per <= 163840 && ncoil >= 2) ? 2 : 1;
+    if (g < 2) return (2 * per <= 131072 && ncoil >= 2) ? 2 : 1;
     g &= ~1LL;
     if (g > ncoil) g = ncoil;
     while (g > 2 && rows * mr_ceil_div(ncoil, g) < 512) g = (g + 1) / 2;

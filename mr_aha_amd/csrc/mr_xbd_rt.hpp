@@ -4,7 +4,8 @@
 #include "mr_hip.hpp"
 
 // LDS values per work-item of a workgroup: 512 work-items hold 80 KB of
-// pencils (two workgroups per CU), 1024 hold 160 KB (one).
+// pencils (two workgroups per CU), 1024 have room for 160 KB (one) and are given
+// up to 128 KB (MR_XBD_EMAX values).
 #define MR_RT_EPT 20
 #define MR_RT_MAXST 16
 
