@@ -547,12 +547,12 @@ def main():
             stages[name] = {"avg_ms": round(avg, 4), "launches": int(calls[i]),
                             "gbs": round(nb / (avg * 1e6), 1) if nb else None}
     dom = max((s for s in stages if s in sb), key=lambda s: stages[s]["avg_ms"])
-    ct_axis = {256, 320, 384, 512, 640, 56}
     if dom == "BD":
         dom_kernel = ({2: "mr_k_xbd_pd"}.get(xbd_form, "mr_k_xbd_ct") if xbd
-                      else ("mr_k_bd" if cfg.L <= 16 else "mr_k_bdt"))
+                      else ("mr_k_bd" if cfg.L <= 16 else "mr_k_bdm"))
     else:
-        dom_kernel = "mr_fft_axis_ct" if set(cfg.phi2_dim[1:]) <= ct_axis else "mr_fft_axis_fast"
+        # 2D: the inverse outer pass; the grids of the other workloads take the compiled lengths
+        dom_kernel = "mr_k_axis_io" if w["traj_type"] == "2D" and dom == "I2" else "mr_fft_axis_ct"
     dom_ms = stages[dom]["avg_ms"]
     achieved = sb[dom] / (dom_ms * 1e6)
     B = apply_model_bytes(cfg)

@@ -869,12 +869,14 @@ static int mr_blockdiag(mr_aha_plan p, float2 *K, int nc, const float2 *ker)
 
 constexpr int MR_ZD_LB = 8;              // ranks per tile
 // up to this length two workgroups per CU, by LDS and 64 registers (224x224x16,
-// L=8, 10 coils 2.74 -> 2.61 ms, x24 3.99 -> 3.90; 32 spills and gains nothing)
+// L=8, 10 coils 2.74 -> 2.61 ms, x24 3.99 -> 3.90, two registers of the forward
+// kernels spilled; 32 spills more and gains nothing)
 constexpr int MR_ZD_TWO = 24;
 constexpr int MR_ZD_PT = 16 * MR_ZD_LB;  // pencils per tile
 // All twiddles of a butterfly, from the table: in scalar registers they cost no
 // more than the first with its powers, and the apply's error against FP64 falls
-// (320x320x56, L=16, 12 coils 4.1e-7 -> 3.5e-7; at equal speed, 39.3 -> 39.2 ms).
+// (320x320x56, L=16, 12 coils 4.1e-7 -> 3.5e-7; forward pass 2.43 ms both ways,
+// inverse 2.62 -> 2.65).
 constexpr int MR_ZD_WN = 7;
 // LDS stride of one rank's N rows of 16 xy, padded by one row so that the
 // four ranks a wavefront reads at once start on alternate bank halves

@@ -1,6 +1,10 @@
 // Block multiply for ranks above the compiled ones (L = 17 .. 512) where the
 // matrix-core kernel (mr_bdm.hip) does not apply: ranks above 80, and lower ones
-// with few coils. In place over the padded k-space grids of the separate-pass
+// with few coils or, at ranks 17 to 19, coils that fill its rows of 16 badly. Batches
+// of 6 coils at most: of 8 and 12 they gain 1 % at ranks 17 and 18 with
+// 9 to 11 coils and lose elsewhere (grid 400x400, block stage, 12 against 6: L=17, 9
+// to 11 coils, 244 to 258 and 246 to 262 us, 17 coils 495 and 387, 22 coils 525 and
+// 498, L=96, 12 coils, 4.19 and 4.11 ms). In place over the padded k-space grids of the separate-pass
 // route.
 //
 // Same operation as the reference's tiled kernels

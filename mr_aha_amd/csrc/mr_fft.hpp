@@ -9,9 +9,9 @@
 // (Govindaraju et al., "High performance discrete Fourier transforms on
 // graphics processors", SC 2008). Radices 2, 3, 4, 5, 7, 8 have unrolled
 // butterflies, and 6 and 10 prime-factor ones (no internal twiddles, so
-// e.g. 640 = 8 * 8 * 10 takes three stages); any other prime factor uses a
-// per-output dot product over
-// the n-th-root table, so every length works (prime grids of the test
+// e.g. 640 = 8 * 8 * 10 takes three stages); any other prime factor takes
+// half-length cosine and sine sums over the n-th-root table (mr_stage_odd), so
+// every length works (prime grids of the test
 // fixtures) while smooth lengths take the fast butterflies.
 //
 // The transform is unnormalised; FWD uses e^{-2 pi i jk/n}, INV e^{+...}.

@@ -126,12 +126,14 @@ __global__ void mr_k_toep_store(const double2 *nat, int m0, int m1, int m2, int 
 // first M places (the pitch stays that of the fine grid, no second buffer).
 // Later axes then run over M instead of nf values of the finished ones.
 //
-// The bound is memory: 2D moves 16 nf^2 read, 8 nf^2 written and read, 2 nf^2
+// What counts is memory traffic: 2D moves 16 nf^2 read, 8 nf^2 written and read, 2 nf^2
 // written bytes (and the spread's 16 nf^2) where the separate passes moved
 // three times that. Measured, all separate passes and these: 256x256 L=8 (36
 // components, nf 1024) 1.42 -> 0.55 ms, 192x192x32 L=8 (1152, nf 768) 27.3 ->
-// 9.8 ms, 96^3 L=4 (10, nf 384) 27.1 -> 8.3 ms; 2.7 to 3.3 TB/s along x. The pencils of a workgroup share 8 NT values of LDS
-// (72 KB at 512 work-items: two workgroups per CU); along y and z they are neighbours in
+// 9.8 ms, 96^3 L=4 (10, nf 384) 27.1 -> 8.3 ms; 2.7 to 3.2 TB/s along x, 1.8 to
+// 2.8 along y and z. Neither memory nor VALU issue (47 to 58 %) is saturated: a
+// workgroup loads, transforms and stores one after another, and a CU holds two. The
+// pencils of a workgroup share 8 NT values of LDS (72 KB at 512 work-items); along y and z they are neighbours in
 // x, 64 bytes at nf = 1024, and the tiles that share a line are neighbours on
 // one XCD.
 // ---------------------------------------------------------------------------

@@ -21,16 +21,20 @@
 // Padded k-space never reaches HBM: per row and coil the pass moves 2*L*Nx
 // values plus the kernel row.
 //
-// What bounds it is VALU and LDS issue, as in the compiled-length kernels, so
-// it takes over what it can of them at a run-time length: the coil-pair walks
-// with two entries per 16-byte load, the half-empty first stage and the cropped last one where the image fills the
+// What it spends its time on is VALU and LDS issue, one phase after another (55 and
+// 36 % of its cycles at 240x216x40, 15 points of the latter bank conflicts), so
+// it takes over what it can of the compiled-length kernels: the coil-pair walks
+// with two entries per 16-byte load (unmasked kernels), the half-empty first stage
+// and the cropped last one where the image fills the
 // centred half of the pencil, divisions as one full-rate 24-bit multiply,
 // 16-byte image loads and stores. Every twiddle is read from the table (the
-// compiled kernels form powers of one, which is a little less exact). What stays is an add per LDS access (the
-// butterfly strides are not immediates). Measured against the kernel before
-// it (one coil per walk, 8-byte entries, all eight inputs read): 240x216x40,
+// compiled kernels form powers of one, which is a little less exact). What stays is
+// an add per LDS access (the butterfly strides are not immediates). Measured against
+// the kernel before it (one coil per walk, 8-byte entries, all eight inputs read): 240x216x40,
 // grid 480x432x40, L=6, 10 coils, masked 5.66 -> 3.11 ms (5.1 GB, 1.6 TB/s);
-// 225x198, grid 450x396, L=5, 7 coils 91 -> 65 us.
+// 225x198, grid 450x396, L=5, 7 coils 91 -> 65 us. Ranks 14 to 16 spill 4 to 36
+// registers (20 to 96 bytes of scratch a lane) and are faster all the same: 112x96x12, 8
+// coils, L=14, 15, 16: 731 -> 539, 792 -> 574, 867 -> 693 us.
 
 #pragma once
 
