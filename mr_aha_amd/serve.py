@@ -97,8 +97,10 @@ def build_bytes(req: Request) -> int:
     strengths of the Gram blocks, per sample its sort keys (twice), indexes
     (twice), first points, readout and 16 weights an axis, and the sort's own
     work; blocks may be an eighth larger than asked for, and whole megabytes."""
-    chunk = max(BUILD_BYTES, _build_component_bytes(req))
     ntraj, nkx = int(req.traj.shape[-1]), int(req.traj.shape[-2])
+    # one component, when it is larger than the chunk, with its partial tiles: one of
+    # 64 values per 256 candidates, a sample being one of up to 125 tiles
+    chunk = max(BUILD_BYTES, _build_component_bytes(req) + ntraj * nkx * 125 * 4)
     planes = req.n_dim[2] if req.traj_type == "stack" else 1
     strengths = req.L * (req.L + 1) // 2 * planes * ntraj * 16
     axes = 3 if req.traj_type == "3D" else 2
