@@ -7,6 +7,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
+MB = 1 << 20
 
 
 @pytest.fixture(scope="module")
@@ -37,8 +38,13 @@ def _free():
 
 
 def test_idle_scratch_goes_back(mr):
-    """Builds of two sizes leave at most 4 GiB idle; releasing returns exactly
-    that to the device, and the next builds equal the first."""
+    """Builds of two sizes leave at most 4 GiB idle; releasing returns it to the
+    device, and the next builds equal the first.
+
+    The device counts free memory in pages: blocks of whole megabytes have theirs
+    to themselves, smaller ones share theirs with other allocations and may not
+    show. All of a build's 15 blocks but the fine grids and the weights can be
+    that small, so two builds have fewer than 26 MB of those."""
     mr.release_scratch()
     assert mr.idle_scratch() == 0
     cases = [("2D", (160, 144), 6), ("stack", (64, 48, 12), 4)]
@@ -53,7 +59,7 @@ def test_idle_scratch_goes_back(mr):
     assert 0 < idle <= 4 << 30
     assert mr.release_scratch() == idle
     assert mr.idle_scratch() == 0 and mr.release_scratch() == 0
-    assert _free() - free >= idle
+    assert _free() - free > idle - 26 * MB > 26 * MB
     for a, b in zip(first, build()):
         assert torch.equal(torch.view_as_real(a), torch.view_as_real(b))
     assert mr.idle_scratch() == idle   # the same requests, so the same blocks
